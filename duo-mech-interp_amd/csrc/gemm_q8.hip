@@ -14,7 +14,9 @@
 // (gate, up) row pairs with the neuron pushes applied, writing y[m, n / 2] (fp32, or in the split layout below for
 // down_proj to read without splitting).
 //
-// Two kernels:
+// Three kernels:
+//   gemm_q8_few_kernel (products with too few output tiles to fill the device in the kernels below): 32-row tiles,
+//     the waves of a block split K; see its comment and gemm_few_tile.
 //   gemm_q8_dma_kernel (N >= 2048, K <= 2048: the gate/up and input projections): 128 x 256 tiles, one block of 8
 //     waves per CU, each wave a 64 x 64 output tile. x (fp32) and W (int8) go global -> LDS by DMA (global_load_lds,
 //     no registers) in four stages of 32 K. What bounds this product on MI355X is VALU issue and the matrix core's
@@ -35,9 +37,9 @@
 // rounded the same way). Both kernels then skip the split: the DMA kernel copies the 16-byte hi and lo pieces
 // straight into the planes its A fragments are read from (no fp32 stage, no conversion pass), the register-staged
 // kernel stores the loaded pieces as they are. The products, and so y, are bitwise those of the fp32 input.
-// bf16 input (q35_gemm_q8_bf16, the attention output): hi = x exactly and lo = 0, so the register-staged kernel
-// issues only the hi products (the skipped products are exact zeros): bitwise the product of x.float() wherever the
-// fp32 input also runs the register-staged kernel (N < 2048 or K > 2048); for the wide shapes the fp32 input runs the
+// bf16 input (q35_gemm_q8_bf16, the attention output): hi = x exactly and lo = 0, so the few-row and register-staged
+// kernels issue only the hi products (the skipped products are exact zeros): bitwise the product of x.float() wherever the
+// fp32 input runs the same kernel (N < 2048 or K > 2048); for the wide shapes the fp32 input may run the
 // DMA kernel, whose MFMAs group K differently, and the two agree to fp32 rounding.
 #include <type_traits>
 
@@ -49,6 +51,7 @@ namespace q35 {
 constexpr int kGN = 128;  // output columns per block (register-staged kernel)
 constexpr int kGK = 64;   // K step (register-staged kernel)
 constexpr int kQK = 32;   // K per pipeline stage (DMA kernel)
+constexpr int kFewGroups = 32;  // groups of 128 inputs whose scales a block of the few-row kernel holds (K <= 4096)
 
 enum GemmEpi : int { kGemmStore = 0, kGemmAccumulate = 1, kGemmSwiglu = 2, kGemmSwigluSplit = 3 };
 
@@ -575,9 +578,314 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_rs_kernel(const float* __restr
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Few-row kernel: a block of NW waves owns 32 MT x 32 NT outputs, and its waves split K, so that a product with few
+// output tiles still puts waves and loads on every CU (the tiled kernels give a 111-row product 28 blocks for gate/up
+// and 16 for down_proj). Each wave stages its own K range, no block barrier in the loop: a stage is 32 inputs, its x
+// and W tiles DMA'd into LDS (NS stages per wave, NS - 1 in flight; the loop issues no other vector memory load, so
+// the vmcnt waits count only the DMA stream). Straight-to-register fragment loads were measured first: every lane
+// touches another row's cache line, about 90 cycles per 1 KB wave load on a CU, 15.9-28 us for the 111-row gate/up.
+// x is re-read by every block of a row panel through L2, which bounds the kernel. The waves' sums meet in LDS, each in
+// its own stage area, and are added in wave order (fixed order, as the tiled kernels).
+// whether the column tiles are dealt to the XCDs (evenly to within an eighth)
+__host__ __device__ constexpr bool gemm_few_by_xcd(int64_t N, int BN) {
+  return (N + BN - 1) / BN % 8 == 0 || (N + BN - 1) / BN >= 64;
+}
+
+template <int MT, int NT, int NW, int NS, int EPI, bool GS, int XF>
+__global__ __launch_bounds__(64 * NW) void gemm_q8_few_kernel(const float* __restrict__ X, int64_t ldx,
+                                                              const int8_t* __restrict__ W,
+                                                              const float* __restrict__ ws, float* __restrict__ Y,
+                                                              int64_t ldy, int M, int N, int K,
+                                                              const q35_push* __restrict__ pushes, int npush, int T,
+                                                              int moff, int ys, GemmCap cap) {
+  constexpr int BM = 32 * MT, BN = 32 * NT;
+  constexpr int XB = XF == 2 ? 64 : 128;              // bytes of a staged row of x (32 inputs)
+  constexpr int XI = MT * 32 * XB / 1024;             // DMA instructions (1 KB) of a stage's x; one per 32 columns of W
+  constexpr int SI = XI + NT;
+  constexpr int SB = SI * 1024;                       // bytes per stage: x rows, then W rows of 32 bytes
+  constexpr int RX = 1024 / XB, LX = 64 / RX;         // rows per DMA instruction of x, lanes per row
+  static_assert(NS == 2 || NS == 3, "the waits at the end of a wave's stages");
+  static_assert(NS * SB >= MT * NT * 4096, "the stages hold the wave's sums");
+  __shared__ __attribute__((aligned(16))) char smem[NW][NS * SB];
+  __shared__ float gscale[GS ? kFewGroups * BN : 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, lh = lane >> 5;
+  // block b runs on XCD b % 8: an XCD takes every eighth column tile, with all of its row tiles one after the other,
+  // so that W is read into one L2 only (x, read into every L2, is small here). With few column tiles that would leave
+  // XCDs idle (the 32 last columns of the GDN input projection: one tile), so those go row tiles first over the XCDs.
+  const int mtiles = (M + BM - 1) / BM;
+  int bm, bn;
+  if (gemm_few_by_xcd(N, BN)) {
+    const int at = (int)(blockIdx.x >> 3);
+    bm = at % mtiles;
+    bn = at / mtiles * 8 + (int)(blockIdx.x & 7);
+  } else {
+    bm = (int)blockIdx.x % mtiles;
+    bn = (int)blockIdx.x / mtiles;
+  }
+  const int m0 = bm * BM, n0 = bn * BN;
+  if (n0 >= N) return;
+  // this wave's stages
+  const int KS = K / 32;
+  const int s0 = (int)((int64_t)wave * KS / NW), s1 = (int)((int64_t)(wave + 1) * KS / NW);
+  // DMA sources of this lane (32-bit byte offsets; the launcher keeps x and W under 4 GB). A row's 16-byte chunks are
+  // swizzled so that 16 consecutive lanes reading one chunk of 16 consecutive rows hit 16 distinct 16-byte slots of a
+  // 256-byte window: chunk c of row r at c ^ ((r / 2) % 8) (rows of 128 B), c ^ ((r / 4) % 4) (64 B), c ^ ((r / 8) % 2)
+  // (32 B).
+  uint32_t xsrc[XI], wsrc[NT];
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int row = RX * i + lane / LX;
+    const int c = (lane % LX) ^ (XF == 2 ? (row >> 2) & 3 : (row >> 1) & 7);
+    xsrc[i] = (uint32_t)((size_t)min(m0 + row, M - 1) * ldx * (XB / 32) + 16 * c);
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int row = lane >> 1;
+    wsrc[nt] = (uint32_t)((size_t)min(n0 + 32 * nt + row, N - 1) * K + 16 * ((lane & 1) ^ ((row >> 3) & 1)));
+  }
+  char* const mine = smem[wave];
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(gemm_lds_u32(mine));
+  auto issue = [&](int s, int buf) {
+    const uint32_t base = lds0 + buf * SB;
+    const char* xs = reinterpret_cast<const char*>(X) + (size_t)s * XB;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) gemm_dma16s(xs, xsrc[i], base + i * 1024);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) gemm_dma16s(W + (size_t)s * 32, wsrc[nt], base + (XI + nt) * 1024);
+  };
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (s0 + i < s1) issue(s0 + i, i);
+  if constexpr (GS) {
+    // the block's group scales [group][column], loaded behind the first stages
+    const int G = K >> 7;
+    for (int i = tid; i < G * BN; i += 64 * NW) {
+      const int c = i / G, g = i - c * G;
+      gscale[g * BN + c] = ws[(size_t)min(n0 + c, N - 1) * G + g];
+    }
+    lds_barrier();
+  }
+  // fragment offsets: the lane's inputs of a stage are 16 lh .. 16 lh + 15, 8 for each of the two k steps (x and W
+  // share that order of k); rows 32 apart have the same swizzle
+  uint32_t aoff[2][XF == 2 ? 1 : 2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if constexpr (XF == 2) {
+      aoff[j][0] = (uint32_t)(l32 * 64 + (((2 * lh + j) ^ ((l32 >> 2) & 3)) << 4));
+    } else {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) aoff[j][p] = (uint32_t)(l32 * 128 + (((2 * (2 * lh + j) + p) ^ ((l32 >> 1) & 7)) << 4));
+    }
+  }
+  const uint32_t boff = (uint32_t)(XI * 1024 + l32 * 32 + ((lh ^ ((l32 >> 3) & 1)) << 4));
+  f32x16 acc[MT][NT], gacc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      acc[mt][nt] = zero16();
+      gacc[mt][nt] = zero16();
+    }
+  int buf = 0;
+  for (int s = s0; s < s1; ++s) {
+    // every read of the buffer handed to stage s + NS - 1 has returned; then wait until stage s has landed
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (s + NS - 1 < s1) {
+      issue(s + NS - 1, buf == 0 ? NS - 1 : buf - 1);
+      gemm_wait_vm<(NS - 1) * SI>();
+    } else if (s + 1 < s1) {  // (NS 3: the one stage after s)
+      gemm_wait_vm<SI>();
+    } else {
+      gemm_wait_vm<0>();
+    }
+    const char* st = mine + buf * SB;
+    u32x4 wr[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) wr[nt] = *reinterpret_cast<const u32x4*>(st + boff + nt * 1024);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      bf16x8 w[NT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) w[nt] = i8tobf(wr[nt][2 * j], wr[nt][2 * j + 1]);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const char* xa = st + mt * 32 * XB;
+        bf16x8 hi, lo;
+        if constexpr (XF == 0) {
+          split8(*reinterpret_cast<const f32x4*>(xa + aoff[j][0]), *reinterpret_cast<const f32x4*>(xa + aoff[j][1]), hi,
+                 lo);
+        } else if constexpr (XF == 1) {
+          hi = *reinterpret_cast<const bf16x8*>(xa + aoff[j][0]);
+          lo = *reinterpret_cast<const bf16x8*>(xa + aoff[j][1]);
+        } else {
+          hi = *reinterpret_cast<const bf16x8*>(xa + aoff[j][0]);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          f32x16& d = GS ? gacc[mt][nt] : acc[mt][nt];
+          d = mfma32(hi, w[nt], d);
+          if constexpr (XF != 2) d = mfma32(lo, w[nt], d);
+        }
+      }
+    }
+    if constexpr (GS) {
+      if ((s & 3) == 3 || s + 1 == s1) {  // end of a group of 128 inputs, or of the wave's part of it
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          const float sc = gscale[(s >> 2) * BN + 32 * nt + l32];
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mt][nt][r] += sc * gacc[mt][nt][r];
+            gacc[mt][nt] = zero16();
+          }
+        }
+      }
+    }
+    buf = buf + 1 == NS ? 0 : buf + 1;
+  }
+  // the wave's sums into its own stage area. LDS order of a 32-column tile: row r at (r / 8) 256 + (r % 4) 64 +
+  // ((r / 4) % 2) 32, so that the two lane halves of an accumulator register (rows 4 apart) fill 64 consecutive floats
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  float* const rw = reinterpret_cast<float*>(mine);
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) rw[nt * BM * 32 + (4 * mt + (r >> 2)) * 256 + (r & 3) * 64 + lane] = acc[mt][nt][r];
+  const bool pushes_here = EPI == kGemmSwiglu && gemm_pushes_touch(pushes, npush, n0 >> 1, (n0 + BN) >> 1);
+  __syncthreads();
+  // a thread finishes 4 columns of a row: a wave instruction covers 8 whole rows of a tile
+  for (int i = tid; i < NT * BM * 8; i += 64 * NW) {
+    const int nt = i / (BM * 8), row = (i >> 3) % BM, c = 4 * (i & 7);
+    const int m = m0 + row, n = n0 + 32 * nt + c;
+    const int at = nt * BM * 32 + (row >> 3) * 256 + (row & 3) * 64 + ((row >> 2) & 1) * 32 + c;
+    f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(smem[0]) + at);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(smem[w]) + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += o[e];
+    }
+    if (m >= M) continue;
+    if constexpr (!GS) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= ws[min(n + e, N - 1)];
+    }
+    if constexpr (EPI == kGemmSwiglu) {
+#pragma unroll
+      for (int p2 = 0; p2 < 2; ++p2) {
+        const int nn = n + 2 * p2;
+        if (nn + 1 >= N) break;
+        const int neuron = nn >> 1;
+        float a = gemm_silu(v[2 * p2]) * v[2 * p2 + 1];
+        if (pushes_here) {
+          const int prow = gemm_push_row(moff + m, T);
+          for (int p = 0; p < npush; ++p) a = gemm_push(pushes + p, neuron, prow, a);
+        }
+        gemm_store_act(Y + (int64_t)m * ldy + gemm_act_col(neuron, ys), neuron, a, ys);
+        gemm_capture(cap, moff + m, T, neuron, a);
+      }
+    } else {
+      float* dst = Y + (int64_t)m * ldy + n;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) dst[e] = EPI == kGemmAccumulate ? dst[e] + v[e] : v[e];
+    }
+  }
+}
+
 }  // namespace q35
 
 namespace q35 {
+
+template <int MT, int NT, int NW, int NS, int XF>
+static int gemm_few_launch(const float* x, int64_t ldx, const int8_t* W, const float* w_scale, float* y, int64_t ldy,
+                           int64_t M, int64_t N, int64_t K, int epilogue, bool gs, const q35_push* pushes,
+                           int64_t npush, int64_t T, int64_t moff, int ys, const GemmCap& cap, hipStream_t st) {
+  const int64_t nt = (N + 32 * NT - 1) / (32 * NT);
+  const int64_t nblocks = ((M + 32 * MT - 1) / (32 * MT)) * (gemm_few_by_xcd(N, 32 * NT) ? (nt + 7) / 8 * 8 : nt);
+#define Q35_GEMM_FEW(E, G)                                                                                          \
+  hipLaunchKernelGGL((gemm_q8_few_kernel<MT, NT, NW, NS, E, G, XF>), dim3((unsigned)nblocks), dim3(64 * NW), 0, st, \
+                     x, ldx, W, w_scale, y, ldy, (int)M, (int)N, (int)K, pushes, (int)npush, (int)T, (int)moff, ys,   \
+                     cap)
+  if (gs) {
+    if (epilogue == kGemmStore) Q35_GEMM_FEW(kGemmStore, true);
+    else if (epilogue == kGemmAccumulate) Q35_GEMM_FEW(kGemmAccumulate, true);
+    else Q35_GEMM_FEW(kGemmSwiglu, true);
+  } else {
+    if (epilogue == kGemmStore) Q35_GEMM_FEW(kGemmStore, false);
+    else if (epilogue == kGemmAccumulate) Q35_GEMM_FEW(kGemmAccumulate, false);
+    else Q35_GEMM_FEW(kGemmSwiglu, false);
+  }
+#undef Q35_GEMM_FEW
+  return hipGetLastError() == hipSuccess ? Q35_OK : Q35_ELAUNCH;
+}
+
+// compute units of the current device (the DMA kernel runs one block per CU)
+static int64_t gemm_cu_count() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 256;
+  return cus;
+}
+
+// The few-row kernel's tile for a product, 0 where the tiled kernels are faster. `wide`: the DMA kernel would run it.
+// Measured on MI355X (group scales, weights cycled past the L2, us; gate_up 7168 x 1024, down 1024 x 3584, gdn_in
+// 8224 x 1024, attn_in 5120 x 1024):
+//   1  32 x 32, 8 waves: one block per CU, the shortest K run per wave; best while its blocks fit one round (gate_up
+//      9 rows 5.7 against 6.8 for tile 2 and 31.2 tiled; down 200 rows 12.3, 14.9, 54.7).
+//   2  32 x 64, 8 waves: half the re-reads of x; best while its blocks fit one round (gate_up 64 rows 8.3 against 9.5
+//      for tile 3 and 10.0 for tile 1; down 500 rows 19.5, 23.2, 27.2; 65.4 tiled).
+//   3  32 x 64, 4 waves, two blocks per CU: more than one round, against the DMA kernel (which takes the same time up
+//      to about 700 rows, one round of tiles). gate_up 200 / 300 / 400 / 500 rows 20.9 / 26.2 / 31.2 / 35.5 against
+//      37.6 / 37.9 / 38.4 / 38.6; gdn_in 200 / 300 / 400 rows 20.8 / 28.0 / 33.3 against 30.2 / 31.0 / 31.6; attn_in
+//      500 / 700 rows 25.6 / 34.1 against 30.5 / 31.4: the lines cross at about 1400 blocks.
+//   4  64 x 64, 4 waves: more than one round of tile 2, against the register-staged kernel, while its blocks fit one
+//      round (down 700 / 1000 rows 32.8 / 33.8 against 34.2 / 39.7 for tile 3 and 66.1 / 66.4).
+static int gemm_few_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int xbytes, bool wide) {
+  if (K > 128 * kFewGroups || ((M - 1) * ldx + K) * xbytes > 0xffffffffLL || N * K > 0xffffffffLL) return 0;
+  const int64_t cus = gemm_cu_count();
+  const int64_t m32 = (M + 31) / 32, n64 = (N + 63) / 64;
+  if (m32 * ((N + 31) / 32) <= cus) return 1;
+  if (m32 * n64 <= cus) return 2;
+  if (wide) return m32 * n64 <= 5 * cus + cus / 4 ? 3 : 0;
+  return ((M + 63) / 64) * n64 <= cus ? 4 : 0;
+}
+
+// a product by the few-row kernel where that is the faster one, else by the register-staged kernel
+template <int XF>
+static int gemm_rs_launch(const float* x, int64_t ldx, const int8_t* W, const float* w_scale, float* y, int64_t ldy,
+                          int64_t M, int64_t N, int64_t K, int epilogue, bool gs, const q35_push* pushes, int64_t npush,
+                          int64_t T, int64_t moff, int ys, const GemmCap& cap, hipStream_t st);
+
+template <int XF>
+static int gemm_small_launch(const float* x, int64_t ldx, const int8_t* W, const float* w_scale, float* y, int64_t ldy,
+                             int64_t M, int64_t N, int64_t K, int epilogue, bool gs, const q35_push* pushes,
+                             int64_t npush, int64_t T, int64_t moff, int ys, const GemmCap& cap, hipStream_t st,
+                             int tile) {
+  switch (tile) {
+    case 1:
+      return gemm_few_launch<1, 1, 8, 3, XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, moff,
+                                             ys, cap, st);
+    case 2:
+      return gemm_few_launch<1, 2, 8, 2, XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, moff,
+                                             ys, cap, st);
+    case 3:
+      return gemm_few_launch<1, 2, 4, 3, XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, moff,
+                                             ys, cap, st);
+    case 4:
+      return gemm_few_launch<2, 2, 4, 3, XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, moff,
+                                             ys, cap, st);
+    default:
+      return gemm_rs_launch<XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, moff, ys, cap, st);
+  }
+}
 
 template <int XF>
 static int gemm_rs_launch(const float* x, int64_t ldx, const int8_t* W, const float* w_scale, float* y, int64_t ldy,
@@ -629,15 +937,6 @@ static int gemm_dma_launch(const float* x, int64_t ldx, const int8_t* W, const f
   return hipGetLastError() == hipSuccess ? Q35_OK : Q35_ELAUNCH;
 }
 
-// compute units of the current device (the DMA kernel runs one block per CU)
-static int64_t gemm_cu_count() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
-}
-
 }  // namespace q35
 
 namespace q35 {
@@ -668,11 +967,12 @@ static int gemm_q8_run(const float* x, int64_t ldx, const int8_t* W, int w_dtype
   if (K % kGK != 0 || ldx % (XB ? 8 : 4) != 0 || ((uintptr_t)x & 15) || ((uintptr_t)W & 15)) return Q35_EUNSUPPORTED;
   if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return Q35_EUNSUPPORTED;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // bf16 x: the register-staged kernel (one product per tile: the lo parts are zero)
-  if constexpr (XB)
-    return gemm_rs_launch<2>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, 0, ys, cap, st);
-  // wide products with K <= 2048 (and x, W addressable with 32-bit byte offsets): the DMA kernel
-  if (N >= 2048 && K <= 128 * kDGS && ((M - 1) * ldx + K) * 4 <= 0xffffffffLL && N * K <= 0xffffffffLL) {
+  // wide products with K <= 2048 (and x, W addressable with 32-bit byte offsets) run the DMA kernel, unless x is bf16
+  const bool wide =
+      !XB && N >= 2048 && K <= 128 * kDGS && ((M - 1) * ldx + K) * 4 <= 0xffffffffLL && N * K <= 0xffffffffLL;
+  constexpr int xb = XB ? 2 : 4, XF = XB ? 2 : XS ? 1 : 0;
+  const int tile = gemm_few_tile(M, N, K, ldx, xb, wide);
+  if (wide && tile == 0) {
     // One block per CU, so a last round of blocks that is mostly empty costs as much as a full one. A partial last
     // column tile that costs a whole extra round (the GDN input projection: 8192 + 32 columns) runs on the
     // register-staged kernel after the full tiles (store and accumulate epilogues: their columns are independent);
@@ -696,17 +996,18 @@ static int gemm_q8_run(const float* x, int64_t ldx, const int8_t* W, int w_dtype
     int r = gemm_dma_launch<XS>(x, ldx, W, w_scale, y, ldy, Md, Nd, K, epilogue, gs, pushes, npush, T, ys, cap, st);
     if (r != Q35_OK) return r;
     if (Md < M) {
-      r = gemm_rs_launch<(XS ? 1 : 0)>(x + Md * ldx, ldx, W, w_scale, y + Md * ldy, ldy, M - Md, Nd, K, epilogue, gs,
-                                       pushes, npush, T, Md, ys, cap, st);
+      r = gemm_small_launch<XF>(x + Md * ldx, ldx, W, w_scale, y + Md * ldy, ldy, M - Md, Nd, K, epilogue, gs, pushes,
+                                npush, T, Md, ys, cap, st, gemm_few_tile(M - Md, Nd, K, ldx, xb, true));
       if (r != Q35_OK) return r;
     }
     if (Nd < N)
-      r = gemm_rs_launch<(XS ? 1 : 0)>(x, ldx, W + Nd * K, w_scale + (gs ? Nd * (K / 128) : Nd), y + Nd, ldy, M,
-                                       N - Nd, K, epilogue, gs, pushes, npush, T, 0, ys, cap, st);
+      r = gemm_small_launch<XF>(x, ldx, W + Nd * K, w_scale + (gs ? Nd * (K / 128) : Nd), y + Nd, ldy, M, N - Nd, K,
+                                epilogue, gs, pushes, npush, T, 0, ys, cap, st,
+                                gemm_few_tile(M, N - Nd, K, ldx, xb, false));
     return r;
   }
-  return gemm_rs_launch<(XS ? 1 : 0)>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, 0, ys, cap,
-                                      st);
+  return gemm_small_launch<XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, 0, ys, cap, st,
+                               tile);
 }
 
 }  // namespace q35

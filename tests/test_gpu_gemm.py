@@ -210,3 +210,45 @@ def test_gemm_q8_bf16_input_equals_fp32_input(M, N, K):
     else:
         assert oracle.rel_err(b.cpu(), a.cpu()) <= 1e-5 and oracle.rel_err(d.cpu(), c.cpu()) <= 1e-5
 
+
+
+# the few-row kernel's tiles (32 x 32, 32 x 64 with 8 and 4 waves, 64 x 64) at their edges: one row past a 32-row tile,
+# ragged columns, waves without any K (K 64 over 8 waves), K runs that start inside a group (K 384 over 8 waves), the
+# largest K it takes and one past it (the register-staged kernel), and the first products past its lines
+@pytest.mark.parametrize("x_form", ["fp32", "split", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(9, 32, 64), (33, 130, 384), (32, 8192, 256), (65, 4094, 1024), (111, 7168, 1024),
+                                   (289, 1022, 3584), (700, 1024, 640), (1060, 1024, 512), (385, 7168, 128),
+                                   (10, 66, 4096), (10, 66, 4224)])
+@pytest.mark.parametrize("gs", [True, False])
+def test_gemm_q8_few_rows(x_form, M, N, K, gs):
+    """Store, accumulate and SwiGLU (pushes over three batch rows) against the fp64 product of the dequantised
+    weights. x = hi + lo drops at most 2^-17 of each value, so the relative error stays under 2^-17 + the fp32 sums'
+    K-deep rounding (1e-5 together); bf16 x has no split error. Two runs are bitwise equal (fixed order of sums)."""
+    if gs and K % 128:
+        pytest.skip("group scales need K a multiple of 128")
+    dev = device()
+    q, s = (_q8g if gs else _q8)(N, K, M + N + K)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(K + M)) * 3.0
+    if x_form == "bf16":
+        x = x.to(torch.bfloat16)
+    xd = x.to(dev)
+    xin = ops.split_activations(xd) if x_form == "split" else xd
+    qd, sd = q.to(dev), s.to(dev)
+    ref = x.double() @ omlp.q8_dequant(q, s).double().T
+    announce(f"gemm_q8 few rows {x_form} M{M} N{N} K{K} gs {gs}")
+    y = ops.gemm_q8(xin, qd, sd)
+    assert oracle.rel_err(y.cpu(), ref) <= 1e-5
+    assert torch.equal(y, ops.gemm_q8(xin, qd, sd))
+    base = torch.randn(M, N, generator=torch.Generator().manual_seed(3))
+    out = base.to(dev)
+    ops.gemm_q8(xin, qd, sd, out=out, epilogue="add")
+    # with one scale per row the scaling may fuse with the add: one rounding of y (2^-24 |y|) apart, and the sum's own
+    d = (out.double() - (base.to(dev).double() + y.double())).abs()
+    assert bool((d <= 2.0 ** -23 * (y.abs() + out.abs()).double()).all())
+    T = (M + 2) // 3
+    pushes = [(3, "add", [1.0, -2.0, 0.5]), (1 << 30, "add", [9.0]), (None, "mul", [0.5, 2.0, 1.0])]
+    a = ops.gemm_q8(xin, qd, sd, epilogue="swiglu", pushes=ops.pack_pushes(pushes, dev), T=T)
+    assert oracle.rel_err(a.cpu(), omlp.swiglu_push(ref[:, 0::2].float(), ref[:, 1::2].float(), pushes, T=T)) <= 1e-5
+    if N % 16 == 0:
+        b = ops.gemm_q8(xin, qd, sd, epilogue="swiglu", pushes=ops.pack_pushes(pushes, dev), T=T, split_out=True)
+        assert torch.equal(b, ops.split_activations(a))
