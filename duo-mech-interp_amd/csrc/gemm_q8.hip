@@ -63,9 +63,12 @@ __device__ __forceinline__ float gemm_silu(float x) { return silu_f(x); }
 // records, unused ones matching no neuron). Uniform: the records are read with scalar loads.
 __device__ __forceinline__ bool gemm_pushes_touch(const q35_push* ps, int npush, int nlo, int nhi) {
   bool any = false;
-  for (int p = 0; p < npush; ++p) {
-    const int pn = ps[p].neuron;
-    any |= pn < 0 || (pn >= nlo && pn < nhi);
+  for (int p0 = 0; p0 < npush; p0 += 8) {  // eight records' loads in flight
+    int pn[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) pn[i] = ps[min(p0 + i, npush - 1)].neuron;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) any |= pn[i] < 0 || (pn[i] >= nlo && pn[i] < nhi);
   }
   return any;
 }
@@ -659,6 +662,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_q8_few_kernel(const float* __res
 #pragma unroll
   for (int i = 0; i < NS - 1; ++i)
     if (s0 + i < s1) issue(s0 + i, i);
+  const bool pushes_here = EPI == kGemmSwiglu && gemm_pushes_touch(pushes, npush, n0 >> 1, (n0 + BN) >> 1);
   if constexpr (GS) {
     // the block's group scales [group][column], loaded behind the first stages
     const int G = K >> 7;
@@ -757,7 +761,6 @@ __global__ __launch_bounds__(64 * NW) void gemm_q8_few_kernel(const float* __res
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) rw[nt * BM * 32 + (4 * mt + (r >> 2)) * 256 + (r & 3) * 64 + lane] = acc[mt][nt][r];
-  const bool pushes_here = EPI == kGemmSwiglu && gemm_pushes_touch(pushes, npush, n0 >> 1, (n0 + BN) >> 1);
   __syncthreads();
   // a thread finishes 4 columns of a row: a wave instruction covers 8 whole rows of a tile
   for (int i = tid; i < NT * BM * 8; i += 64 * NW) {

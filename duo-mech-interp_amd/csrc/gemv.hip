@@ -17,61 +17,20 @@
 // the waves in LDS. Epilogues: store, accumulate into y (the residual add after down_proj), or SwiGLU over interleaved
 // (gate, up) row pairs with the neuron pushes applied (gate_up_proj). With group scales a lane's 16 weights of a K step
 // lie in one group (group 2 step + slot / 8), so the lane scales its partial sum of the step once.
-// TL: a block takes tiles blockIdx.x, blockIdx.x + gridDim.x, ... (the LM head's 9496 tiles run on a capped grid);
+// TL (fp32 weights with more tiles than kGemvMaxBlocks): a block takes tiles blockIdx.x, blockIdx.x + gridDim.x, ...;
 // the next tile's weights are issued before the current tile's products when a wave has one K step per tile (two
 // register sets), else before its reduction.
+// What a block waits for, beside the weights: the x operands go out ahead of the weights and are consumed in straight-line
+// code (consumed in a loop, their wait became a wait for the weights too: gate/up at 3 rows 6.9 -> 6.4 us), rows of x are
+// loaded without a branch each, sums cross lanes by DPP rather than through LDS (5120 x 1024 at 3 rows 5.6 -> 5.3), and
+// whether a push touches the tile is known before the epilogue (gate/up with the model's eight records 8.0 -> 6.2).
 // Split K: an accumulating product without the norm prologue may split its K steps over gridDim.y blocks per 16 rows
 // (a product with few output rows, e.g. N = 1024, has too few blocks to draw bandwidth from every CU); each block
 // stages and reads only its share of x and W and adds its sums into y with fp32 atomics, so the order of the
 // additions, and the last bits of y, may differ between runs.
-#include "q35_common.h"
-#include "q35hip.h"
+#include "gemv_common.h"
 
 namespace q35 {
-
-enum GemvEpi : int { kEpiStore = 0, kEpiAccumulate = 1, kEpiSwiglu = 2, kEpiConv = 3 };
-constexpr int kEpiAccumulateFixed = 4;  // entry-point code: accumulate, every output summed in one fixed order
-constexpr int kGemvConvMaxK = 8;  // conv taps supported by the conv epilogue
-constexpr int kGemvHead = 128;    // head size of the gated-norm prologue
-
-// Operands of the gated-norm prologue (GN) and of the conv epilogue (kEpiConv); unused by the other forms.
-struct GemvAux {
-  const float* z;    // GN: gate rows z[m * ldz + k]
-  int64_t ldz;
-  const float* hs;   // GN: per-head scale (may be NULL)
-  const float* cw;   // conv: weights [cc][ck]
-  const float* cb;   // conv: bias [cc] (may be NULL)
-  float* cst;        // conv: state [M][ck - 1][cc]
-  int cc, ck;        // conv: channels (outputs 0 .. cc - 1 are convolved), taps
-  float* cap;        // SwiGLU: activation capture (may be NULL): row m, neuron n at
-  int64_t ldc, ldcr; //   cap[(m / T) ldcr + (m % T) ldc + n]
-  unsigned long long* amax;  // store: per-row argmax keys (may be NULL), see amax_key
-};
-
-// Argmax key of output n with value v: the order-preserving bits of v above the complement of n, so that the largest
-// key is the largest value and, among equal values, the lowest index (as argmax_rows_kernel and torch.argmax). -0
-// ranks as +0; NaN gets 0, the empty key, and never wins (the scan's strict comparisons). A real key is never 0.
-__device__ __forceinline__ unsigned long long amax_key(float v, int n) {
-  if (!(v == v)) return 0ull;
-  if (v == 0.f) v = 0.f;
-  uint32_t b = __float_as_uint(v);
-  b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-  return ((unsigned long long)b << 32) | (0xFFFFFFFFu - (uint32_t)n);
-}
-
-__device__ __forceinline__ float gsilu(float x) { return silu_f(x); }
-
-// one push applied to activation a of neuron n (fields read straight from the record: no copy of the value array)
-__device__ __forceinline__ float apply_push(const q35_push* ps, int n, int row, float a) {
-  const int pn = ps->neuron;
-  if (pn != n && pn >= 0) return a;
-  const float v = ps->vals[row];
-  return ps->mode ? a * v : a + v;
-}
-
-template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
 
 // 16 bytes of weights as fp32: int8 x 16 or fp32 x 4
 template <typename TW> struct WChunk;
@@ -91,13 +50,11 @@ template <> struct WChunk<float> {
   __device__ __forceinline__ float at(int i) const { return r[i]; }
 };
 
-// sum over the 16 lanes of a DPP row (lanes 16 r .. 16 r + 15), result in every lane of the row
-__device__ __forceinline__ float row16_sum_f(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  return v + dpp_f<0x140>(v);  // row_mirror
-}
+// Where the 16 bytes of staged x at column k (a multiple of 4) lie in their row: a lane of the int8 form reads 64
+// consecutive bytes, so 16 lanes reading one 16-byte piece each at a stride of 64 bytes would share 4 of the 16 slots
+// of a 256-byte window (a 4-way bank conflict); swapping pieces within each 64 bytes by the 256-byte window's 64-byte
+// quarter gives each lane its own slot.
+__device__ __forceinline__ int xs_at(int k) { return k ^ (((k >> 6) & 3) << 2); }
 
 // NORM: x is a residual row; the kernel adds xadd (may be NULL), writes the sum to xout from block 0 (may be NULL),
 // and multiplies the RMSNorm of the sum, s * rsqrt(mean s^2 + eps) * (1 + nw), instead of x (HF:720-734).
@@ -171,8 +128,8 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
       fw = *reinterpret_cast<const f32x4*>(nw + kf);
 #pragma unroll
       for (int m = 0; m < MP; ++m) {
-        if (m < M) fv[m] = *reinterpret_cast<const f32x4*>(x + m * ldx + kf);
-        if (m < M && xadd) fa[m] = *reinterpret_cast<const f32x4*>(xadd + m * ldx + kf);
+        if (MP < 8 || m < M) fv[m] = *reinterpret_cast<const f32x4*>(x + m * ldx + kf);
+        if ((MP < 8 || m < M) && xadd) fa[m] = *reinterpret_cast<const f32x4*>(xadd + m * ldx + kf);
       }
     }
   } else {
@@ -199,6 +156,8 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
       }
     }
   }
+  int pn = 0x7fffffff;
+  if (EPI == kEpiSwiglu) pn = push_neuron(pushes, npush);
   issue(sb + wave);
   // kEpiConv: the epilogue thread of (output row rr, row m) holds its channel's taps, bias and conv state, loaded
   // behind the weights (the epilogue needs the weights' products first anyway)
@@ -224,83 +183,90 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
     float ss[MP];
 #pragma unroll
     for (int m = 0; m < MP; ++m) ss[m] = 0.f;
-    for (int k = kf; k < K; k += 4 * (int)blockDim.x) {
-      const bool first = k == kf;
-      const f32x4 w = first ? fw : *reinterpret_cast<const f32x4*>(nw + k);
-      f32x4 v[MP];
+    auto chunk = [&](int k, const f32x4& w, const f32x4 (&v)[MP], const f32x4 (&a)[MP]) {
 #pragma unroll
       for (int m = 0; m < MP; ++m) {
-        v[m] = zero4();
-        if (m < M) v[m] = first ? fv[m] : *reinterpret_cast<const f32x4*>(x + m * ldx + k);
-      }
-      if (xadd) {
+        f32x4 t = v[m];
+        if (xadd) {
 #pragma unroll
-        for (int m = 0; m < MP; ++m) {
-          if (m < M) {
-            const f32x4 a = first ? fa[m] : *reinterpret_cast<const f32x4*>(xadd + m * ldx + k);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[m][e] += a[e];
-          }
+          for (int e = 0; e < 4; ++e) t[e] += a[m][e];
         }
-      }
-#pragma unroll
-      for (int m = 0; m < MP; ++m) {
-        if (xout && blockIdx.x == 0 && m < M) *reinterpret_cast<f32x4*>(xout + m * ldx + k) = v[m];
+        if (xout && blockIdx.x == 0 && (MP < 8 || m < M)) *reinterpret_cast<f32x4*>(xout + m * ldx + k) = t;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          ss[m] += v[m][e] * v[m][e];
-          v[m][e] *= 1.f + w[e];
+          ss[m] += t[e] * t[e];
+          t[e] *= 1.f + w[e];
         }
-        *reinterpret_cast<f32x4*>(xs + m * K + k) = v[m];
+        *reinterpret_cast<f32x4*>(xs + m * K + xs_at(k)) = t;
       }
+    };
+    // the first chunk outside the loop: inside it, the wait for its operands would merge with the loop's own loads into
+    // a wait for everything, the weights included
+    if (kf < K) chunk(kf, fw, fv, fa);
+    for (int k = kf + 4 * (int)blockDim.x; k < K; k += 4 * (int)blockDim.x) {
+      const f32x4 w = *reinterpret_cast<const f32x4*>(nw + k);
+      f32x4 v[MP], a[MP];
+#pragma unroll
+      for (int m = 0; m < MP; ++m) {
+        v[m] = a[m] = zero4();
+        if (MP < 8 || m < M) v[m] = *reinterpret_cast<const f32x4*>(x + m * ldx + k);
+        if ((MP < 8 || m < M) && xadd) a[m] = *reinterpret_cast<const f32x4*>(xadd + m * ldx + k);
+      }
+      chunk(k, w, v, a);
     }
 #pragma unroll
     for (int m = 0; m < MP; ++m) {
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) ss[m] += __shfl_xor(ss[m], off, 64);
-      if (lane == 0) ssw[wave][m] = ss[m];
+      const float t = wave_sum_f(ss[m]);
+      if (lane == 0) ssw[wave][m] = t;
     }
   } else if (GN) {
     // gated RMSNorm per head of 128 inputs (the fused GDN decode step's order): x * r * w * silu(z) * hs, with
     // r = rsqrt(mean x^2 + eps) over the head. Kb and kb0 are multiples of 128, so the 32 quads of a head are 32
     // consecutive i: one half wave, reduced with shuffles inside it (a half wave is wholly in or out of the loop)
-    for (int j = 0, i = tid; i < MP * Kb / 4; ++j, i += blockDim.x) {
-      const int m = (4 * i) / Kb, k = 4 * i - m * Kb, kk = kb0 + k;
+    auto quad = [&](int i, const f32x4& o, const f32x4& zz, const f32x4& w, float hsc) {
+      const int m = (4 * i) / Kb, k = 4 * i - m * Kb;
+      const float ss = half_sum_f(o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3]);
+      const float r = rsqrtf(ss * (1.f / kGemvHead) + eps);
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = w[e] * (o[e] * r) * gsilu(zz[e]) * hsc;
+      *reinterpret_cast<f32x4*>(xs + m * Kb + xs_at(k)) = v;
+    };
+#pragma unroll
+    for (int q = 0; q < kGnPre; ++q) {  // (the first quads outside the loop, as above)
+      const int i = tid + q * (int)blockDim.x;
+      if (i < MP * Kb / 4) quad(i, go[q], gz[q], gw[q], gh[q]);
+    }
+    for (int i = tid + kGnPre * (int)blockDim.x; i < MP * Kb / 4; i += blockDim.x) {
+      const int m = (4 * i) / Kb, kk = kb0 + 4 * i - m * Kb;
       f32x4 o = zero4(), zz = zero4(), w = zero4();
       float hsc = 1.f;
-      if (j < kGnPre) {
-#pragma unroll
-        for (int jj = 0; jj < kGnPre; ++jj)
-          if (jj == j) { o = go[jj]; zz = gz[jj]; w = gw[jj]; hsc = gh[jj]; }
-      } else if (m < M) {
+      if (m < M) {
         o = *reinterpret_cast<const f32x4*>(x + m * ldx + kk);
         zz = *reinterpret_cast<const f32x4*>(aux.z + m * aux.ldz + kk);
         w = *reinterpret_cast<const f32x4*>(nw + (kk & (kGemvHead - 1)));
         if (aux.hs) hsc = aux.hs[kk / kGemvHead];
       }
-      float ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
-#pragma unroll
-      for (int off = 1; off < 32; off <<= 1) ss += __shfl_xor(ss, off, 64);
-      const float r = rsqrtf(ss * (1.f / kGemvHead) + eps);
-      f32x4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = w[e] * (o[e] * r) * gsilu(zz[e]) * hsc;
-      *reinterpret_cast<f32x4*>(xs + m * Kb + k) = v;
+      quad(i, o, zz, w, hsc);
     }
   } else {
-    for (int i = tid; i < MP * Kb / 4; i += blockDim.x) {
+    auto put = [&](int i, const f32x4& v) {
       const int m = (4 * i) / Kb, k = 4 * i - m * Kb;
-      f32x4 v = zero4();
-      if (m < M) v = i == tid ? fv[0] : *reinterpret_cast<const f32x4*>(x + m * ldx + kb0 + k);
-      *reinterpret_cast<f32x4*>(xs + m * Kb + k) = v;
+      *reinterpret_cast<f32x4*>(xs + m * Kb + xs_at(k)) = v;
+    };
+    if (tid < MP * Kb / 4) put(tid, fv[0]);  // (the first quad outside the loop, as above)
+    for (int i = tid + (int)blockDim.x; i < MP * Kb / 4; i += blockDim.x) {
+      const int m = (4 * i) / Kb, k = 4 * i - m * Kb;
+      put(i, m < M ? *reinterpret_cast<const f32x4*>(x + m * ldx + kb0 + k) : zero4());
     }
   }
   __syncthreads();
   // NORM: row m's rsqrt(mean s^2 + eps) factor (TL: once per block, else in the epilogue)
   auto rs = [&](int m) {
-    float ss = 0.f;
-    for (int w = 0; w < NW; ++w) ss += ssw[w][m];
-    return rsqrtf(ss / (float)K + eps);
+    float t[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) t[w] = w < NW ? ssw[w][m] : 0.f;
+    return rsqrtf((((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) / (float)K + eps);
   };
   float rsf[MP];
   if (NORM && TL) {
@@ -310,6 +276,7 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
   // acc += this wave's K step st over the lane's rows, weights (and group scales) from w (ws)
   auto mac = [&](const WChunk<TW>(&w)[R], const float(&ws)[R], int st, float(&acc)[R][MP]) {
     const int k = (st - sb) * KS + j * E;  // column in the staged x (Kb == K without a split)
+    // (its 16-byte pieces k + c in the order of xs_at)
     float part[R][MP];                     // GS: this step's sums, scaled once by the group's scale
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -319,7 +286,7 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
     for (int c = 0; c < E; c += 4) {
       f32x4 xv[MP];
 #pragma unroll
-      for (int m = 0; m < MP; ++m) xv[m] = *reinterpret_cast<const f32x4*>(xs + m * Kb + k + c);
+      for (int m = 0; m < MP; ++m) xv[m] = *reinterpret_cast<const f32x4*>(xs + m * Kb + xs_at(k + c));
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
 #pragma unroll
@@ -400,6 +367,7 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
       }
     } else {
       // rows 2 q and 2 q + 1 of the tile are gate and up of neuron n0 / 2 + q
+      const bool touched = pushes_touch(pn, n0 >> 1, (n0 >> 1) + 2 * R);
       if (tid < 2 * R * MP) {
         const int qn = tid / MP, m = tid - qn * MP;
         const int ng = n0 + 2 * qn;
@@ -409,7 +377,8 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
           if (wscale && !GS) { gt *= wscale[ng]; up *= wscale[ng + 1]; }
           float a = gsilu(gt) * up;
           const int row = min(m / T, 3);
-          for (int p = 0; p < npush; ++p) a = apply_push(pushes + p, neuron, row, a);
+          if (touched)
+            for (int p = 0; p < npush; ++p) a = apply_push(pushes + p, neuron, row, a);
           y[m * ldy + neuron] = a;
           if (aux.cap) aux.cap[(int64_t)(m / T) * aux.ldcr + (int64_t)(m % T) * aux.ldc + neuron] = a;
         }
@@ -537,27 +506,23 @@ __global__ __launch_bounds__(256) void swiglu_push_kernel(const float* __restric
 
 }  // namespace q35
 
+using q35::GemvArgs;
+
 namespace {
 // Blocks of 16 output rows at which a product is split over K: below this many, an accumulating product without the
 // norm splits its K steps so that blocks x splits reaches it (one block per CU of the MI355X).
 constexpr int64_t kGemvSplitTarget = 256;
-// Grid cap: a product with more 16-row tiles (the LM head: 9496) loops each block over tiles blockIdx.x,
-// + gridDim.x, ... (x staged once per block; four 4-wave blocks per CU at 128 VGPRs). The products with fewer tiles
-// take one tile per block, in a kernel without the loop (measured faster for them).
+// Grid cap: an fp32 product with more 16-row tiles loops each block over tiles blockIdx.x, + gridDim.x, ... (x staged
+// once per block; four 4-wave blocks per CU at 128 VGPRs), an int8 one (the LM head: 9496) runs the tile loop of
+// gemv_mfma.hip. The products with fewer tiles take one tile per block (measured faster for them).
 constexpr int64_t kGemvMaxBlocks = 1024;
-
-struct NormArgs {
-  const float* xadd;
-  const float* nw;
-  float eps;
-  float* xout;
-  q35::GemvAux aux;
-};
+// Rows of x from which an int8 product runs on the matrix core: the times on both sides of the line are in gemv_mfma.hip.
+constexpr int64_t kGemvMfmaRows = 4;
 
 template <typename TW, int EPI, int U, bool NORM, bool GS, bool GN, int R = 4>
 void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale, float* y, int64_t ldy, int64_t M,
                    int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T, int nw, int nsplit,
-                   const NormArgs& na, hipStream_t st) {
+                   const GemvArgs& na, hipStream_t st) {
   using namespace q35;
   const int mp = M <= 1 ? 1 : M <= 2 ? 2 : M <= 3 ? 3 : M <= 4 ? 4 : 8;
   constexpr int KS = 16 * WChunk<TW>::kElems;
@@ -572,30 +537,28 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
   hipLaunchKernelGGL((gemv_kernel<TW, MP, EPI, U, NORM, GS, TL, (MP == 8 ? R8 : R), GN>), grid, block, lds, st, x, \
                      ldx, W, wscale, y, ldy, (int)M, (int)N, (int)K, pushes, npush, (int)T, na.xadd, na.nw, na.eps,   \
                      na.xout, na.aux)
-  if constexpr (EPI == kEpiConv) {  // one tile per block (the entry point bounds N)
-    switch (mp) {
-      case 1: Q35_GEMV(1, false); break;
-      case 2: Q35_GEMV(2, false); break;
-      case 3: Q35_GEMV(3, false); break;
-      case 4: Q35_GEMV(4, false); break;
-      default: if constexpr (U <= 2) Q35_GEMV(8, false); break;  // 8 rows: U <= 2 (gemv_launch)
+  // int8 products of kGemvMfmaRows rows or more, and those with more tiles than blocks, run gemv_mfma.hip; the 4-row
+  // tiles (R 1) stay here for every M
+  constexpr bool kFew = sizeof(TW) == 1 && R > 1;
+  if constexpr (EPI != kEpiConv && !kFew && R > 1) {
+    if (ntiles > kGemvMaxBlocks) {
+      switch (mp) {
+        case 1: Q35_GEMV(1, true); break;
+        case 2: Q35_GEMV(2, true); break;
+        case 3: Q35_GEMV(3, true); break;
+        case 4: Q35_GEMV(4, true); break;
+        default: if constexpr (U <= 2) Q35_GEMV(8, true); break;  // 8 rows: U <= 2 (gemv_launch)
+      }
+      return;
     }
-  } else if (ntiles > kGemvMaxBlocks) {
-    switch (mp) {
-      case 1: Q35_GEMV(1, true); break;
-      case 2: Q35_GEMV(2, true); break;
-      case 3: Q35_GEMV(3, true); break;
-      case 4: Q35_GEMV(4, true); break;
-      default: if constexpr (U <= 2) Q35_GEMV(8, true); break;  // 8 rows: U <= 2 (gemv_launch)
-    }
-  } else {
-    switch (mp) {
-      case 1: Q35_GEMV(1, false); break;
-      case 2: Q35_GEMV(2, false); break;
-      case 3: Q35_GEMV(3, false); break;
-      case 4: Q35_GEMV(4, false); break;
-      default: if constexpr (U <= 2) Q35_GEMV(8, false); break;  // 8 rows: U <= 2 (gemv_launch)
-    }
+  }
+  // one tile per block (the conv epilogue's entry point bounds N)
+  switch (mp) {
+    case 1: Q35_GEMV(1, false); break;
+    case 2: Q35_GEMV(2, false); break;
+    case 3: Q35_GEMV(3, false); break;
+    case 4: if constexpr (!kFew) Q35_GEMV(4, false); break;
+    default: if constexpr (!kFew && U <= 2) Q35_GEMV(8, false); break;  // 8 rows: U <= 2 (gemv_launch)
   }
 #undef Q35_GEMV
 }
@@ -607,7 +570,7 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
 // output is summed in one order whatever the run (0.6-1.4 us slower per call than the split at N = 1024, M = 3)
 template <typename TW, int EPI, bool NORM, bool GS = false, bool GN = false>
 int gemv_launch(const float* x, int64_t ldx, const TW* W, const float* wscale, float* y, int64_t ldy, int64_t M,
-                int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T, const NormArgs& na,
+                int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T, const GemvArgs& na,
                 hipStream_t st, bool fixed = false) {
   using namespace q35;
   const int64_t steps = K / (16 * WChunk<TW>::kElems);
@@ -634,6 +597,10 @@ int gemv_launch(const float* x, int64_t ldx, const TW* W, const float* wscale, f
   const int64_t bsteps = (steps + nsplit - 1) / nsplit;
   const int nw = bsteps <= 4 ? 4 : 8;
   const int64_t per_wave = (bsteps + nw - 1) / nw;
+  if constexpr (sizeof(TW) == 1) {
+    if (M >= kGemvMfmaRows || (EPI != kEpiConv && !GN && nsplit == 1 && nblk > kGemvMaxBlocks))
+      return gemv_mfma_run(NORM, GN, GS, EPI, x, ldx, W, wscale, y, ldy, M, N, K, pushes, npush, T, (int)nsplit, na, st);
+  }
   // more than 4 rows of x: at most two K steps per wave in flight (four spill the registers of 8 rows)
   if (per_wave <= 1)
     gemv_launch_u<TW, EPI, 1, NORM, GS, GN>(x, ldx, W, wscale, y, ldy, M, N, K, pushes, npush, T, nw, (int)nsplit, na, st);
@@ -649,7 +616,7 @@ int gemv_launch(const float* x, int64_t ldx, const TW* W, const float* wscale, f
 template <bool NORM>
 int gemv_dispatch(const float* x, int64_t ldx, const void* W, int w_dtype, const float* w_scale, float* y,
                   int64_t ldy, int64_t M, int64_t N, int64_t K, int epilogue, const q35_push* pushes, int np,
-                  int64_t T, const NormArgs& na, hipStream_t st) {
+                  int64_t T, const GemvArgs& na, hipStream_t st) {
   using namespace q35;
   const bool fx = epilogue == kEpiAccumulateFixed;
   const bool acc = epilogue == kEpiAccumulate || fx;
@@ -699,7 +666,7 @@ extern "C" int q35_gemv(const float* x, int64_t ldx, const void* W, int w_dtype,
   const int chk = gemv_check(x, ldx, W, w_dtype, w_scale, y, ldy, M, N, K, epilogue, pushes, npush, T, cap, ld_cap,
                              ld_cap_row);
   if (chk != Q35_OK) return chk;
-  NormArgs na = {nullptr, nullptr, 0.f, nullptr, {}};
+  GemvArgs na = {nullptr, nullptr, 0.f, nullptr, {}};
   na.aux.cap = cap;
   na.aux.ldc = ld_cap;
   na.aux.ldcr = ld_cap_row;
@@ -722,7 +689,7 @@ extern "C" int q35_gemv_norm(const float* x, const float* x_add, float* x_out, i
     return a && x_out && a < x_out + (M - 1) * ldx + K && x_out < a + (M - 1) * ldx + K;
   };
   if (overlap(x) || overlap(x_add)) return Q35_EINVAL;
-  NormArgs na = {x_add, norm_w, eps, x_out, {}};
+  GemvArgs na = {x_add, norm_w, eps, x_out, {}};
   na.aux.cap = cap;
   na.aux.ldc = ld_cap;
   na.aux.ldcr = ld_cap_row;
@@ -745,7 +712,7 @@ extern "C" int q35_gemv_norm_argmax(const float* x, const float* x_add, float* x
     return a && x_out && a < x_out + (M - 1) * ldx + K && x_out < a + (M - 1) * ldx + K;
   };
   if (overlap(x) || overlap(x_add)) return Q35_EINVAL;
-  NormArgs na = {x_add, norm_w, eps, x_out, {}};
+  GemvArgs na = {x_add, norm_w, eps, x_out, {}};
   na.aux.amax = reinterpret_cast<unsigned long long*>(slots);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int r = gemv_dispatch<true>(x, ldx, W, w_dtype, w_scale, y, ldy, M, N, K, kEpiStore, nullptr, 0, 1, na, st);
@@ -774,7 +741,7 @@ extern "C" int q35_gemv_norm_conv(const float* x, const float* x_add, float* x_o
     return a && x_out && a < x_out + (M - 1) * ldx + K && x_out < a + (M - 1) * ldx + K;
   };
   if (overlap(x) || overlap(x_add)) return Q35_EINVAL;
-  NormArgs na = {x_add, norm_w, eps, x_out, {}};
+  GemvArgs na = {x_add, norm_w, eps, x_out, {}};
   na.aux.cw = conv_w;
   na.aux.cb = conv_bias;
   na.aux.cst = conv_state;
@@ -804,7 +771,7 @@ extern "C" int q35_gemv_gated_norm(const float* o, int64_t ldo, const float* z, 
   // the prologue normalises whole heads of 128 inputs: int8 weights (K steps of 256) keep every split head-aligned
   if (w_dtype == Q35_F32) return Q35_EUNSUPPORTED;
   if ((ldz & 3) || ((uintptr_t)z & 15) || ((uintptr_t)norm_w & 15)) return Q35_EUNSUPPORTED;
-  NormArgs na = {nullptr, norm_w, eps, nullptr, {}};
+  GemvArgs na = {nullptr, norm_w, eps, nullptr, {}};
   na.aux.z = z;
   na.aux.ldz = ldz;
   na.aux.hs = head_scale;

@@ -1,0 +1,99 @@
+// What the decode GEMV's two translation units share: gemv.hip (fp32 FMA) and gemv_mfma.hip (matrix core).
+#pragma once
+#include "q35_common.h"
+#include "q35hip.h"
+
+namespace q35 {
+
+enum GemvEpi : int { kEpiStore = 0, kEpiAccumulate = 1, kEpiSwiglu = 2, kEpiConv = 3 };
+constexpr int kEpiAccumulateFixed = 4;  // entry-point code: accumulate, every output summed in one fixed order
+constexpr int kGemvConvMaxK = 8;  // conv taps supported by the conv epilogue
+constexpr int kGemvHead = 128;    // head size of the gated-norm prologue
+
+// Operands of the gated-norm prologue (GN) and of the conv epilogue (kEpiConv); unused by the other forms.
+struct GemvAux {
+  const float* z;    // GN: gate rows z[m * ldz + k]
+  int64_t ldz;
+  const float* hs;   // GN: per-head scale (may be NULL)
+  const float* cw;   // conv: weights [cc][ck]
+  const float* cb;   // conv: bias [cc] (may be NULL)
+  float* cst;        // conv: state [M][ck - 1][cc]
+  int cc, ck;        // conv: channels (outputs 0 .. cc - 1 are convolved), taps
+  float* cap;        // SwiGLU: activation capture (may be NULL): row m, neuron n at
+  int64_t ldc, ldcr; //   cap[(m / T) ldcr + (m % T) ldc + n]
+  unsigned long long* amax;  // store: per-row argmax keys (may be NULL), see amax_key
+};
+
+// Argmax key of output n with value v: the order-preserving bits of v above the complement of n, so that the largest
+// key is the largest value and, among equal values, the lowest index (as argmax_rows_kernel and torch.argmax). -0
+// ranks as +0; NaN gets 0, the empty key, and never wins (the scan's strict comparisons). A real key is never 0.
+__device__ __forceinline__ unsigned long long amax_key(float v, int n) {
+  if (!(v == v)) return 0ull;
+  if (v == 0.f) v = 0.f;
+  uint32_t b = __float_as_uint(v);
+  b = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+  return ((unsigned long long)b << 32) | (0xFFFFFFFFu - (uint32_t)n);
+}
+
+__device__ __forceinline__ float gsilu(float x) { return silu_f(x); }
+
+// Whether any push record can touch neurons nlo .. nhi - 1 (a record for every neuron, or for one in the range): the
+// model passes eight records per layer, unused ones matching no neuron, and an epilogue that walks them pays one memory
+// round trip per record. Lane p of a wave takes record p (npush <= 64): push_neuron's load goes out ahead of the
+// weights, pushes_touch votes on it in the epilogue.
+__device__ __forceinline__ int push_neuron(const q35_push* ps, int npush) {
+  const int p = threadIdx.x & 63;
+  return p < npush ? ps[p].neuron : 0x7fffffff;
+}
+__device__ __forceinline__ bool pushes_touch(int pn, int nlo, int nhi) {
+  return __any(pn < 0 || (pn >= nlo && pn < nhi));
+}
+
+// one push applied to activation a of neuron n (fields read straight from the record: no copy of the value array)
+__device__ __forceinline__ float apply_push(const q35_push* ps, int n, int row, float a) {
+  const int pn = ps->neuron;
+  if (pn != n && pn >= 0) return a;
+  const float v = ps->vals[row];
+  return ps->mode ? a * v : a + v;
+}
+
+template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+
+// sum over the 16 lanes of a DPP row (lanes 16 r .. 16 r + 15), result in every lane of the row
+__device__ __forceinline__ float row16_sum_f(float v) {
+  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f<0x141>(v);  // row_half_mirror
+  return v + dpp_f<0x140>(v);  // row_mirror
+}
+
+// sum over 32 lanes (lanes 0 .. 31 or 32 .. 63) and over the wave, in every lane: DPP within rows of 16, one lane exchange
+// or scalar reads across rows (six lane exchanges through LDS took longer than the loads they waited for)
+__device__ __forceinline__ float half_sum_f(float v) {
+  v = row16_sum_f(v);
+  return v + __shfl_xor(v, 16, 64);
+}
+__device__ __forceinline__ float wave_sum_f(float v) {
+  v = row16_sum_f(v);
+  auto at = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+  return (at(0) + at(16)) + (at(32) + at(48));
+}
+
+// the prologues' operands (GN: nw is the gated norm's weight) and the epilogues'
+struct GemvArgs {
+  const float* xadd;
+  const float* nw;
+  float eps;
+  float* xout;
+  GemvAux aux;
+};
+
+// The matrix-core form (int8 weights): gemv_mfma.hip. gs: group scales; norm / gn: the RMSNorm and gated-norm prologues
+// (norm also runs the conv epilogue). nsplit > 1: split K over blocks (accumulate). Returns a q35 status.
+int gemv_mfma_run(bool norm, bool gn, bool gs, int epi, const float* x, int64_t ldx, const int8_t* W,
+                  const float* wscale, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K, const q35_push* pushes,
+                  int npush, int64_t T, int nsplit, const GemvArgs& na, hipStream_t st);
+
+}  // namespace q35

@@ -306,3 +306,71 @@ def test_gemv_group_scales_one_and_eight_rows(M, N, K, epi):
     e = oracle.rel_err(got, ref)
     print(f"gemv M{M} N{N} {epi}: rel err {e:.2e}")
     assert e <= TOL
+
+
+# the matrix-core form: every row count it takes, one column tile of pieces (4, 5 rows) and two (6 to 8), a ragged last
+# tile, one K step, waves without a K step, two rounds of K steps (K 2048 at 8 waves; K 1280 in the tile loop, which
+# also ends a round early), more tiles than blocks
+@pytest.mark.parametrize("M", [1, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("N,K", [(17, 256), (1030, 1024), (500, 2048), (16405, 256), (16390, 1280)])
+@pytest.mark.parametrize("gs", [True, False])
+def test_gemv_matrix_core_rows(M, N, K, gs):
+    """Store, accumulate, SwiGLU with pushes, with and without the norm, against fp64. The pieces of x are exact, so the
+    error is that of fp32 sums and of the norm in fp32: under K 2^-24 in the worst case and well under 2e-6 at random
+    signs."""
+    dev = device()
+    g = torch.Generator().manual_seed(N + K + M)
+    w = torch.randn(N, K, generator=g) * 0.02
+    W, s = omlp.q8_quantize(w) if gs else _weights(N, K, torch.int8, seed=N + K)
+    x = torch.randn(M, K, generator=g) * torch.logspace(-3, 3, K)  # (six decades: every piece matters)
+    nw = torch.randn(K, generator=g) * 0.1
+    wd = omlp.q8_dequant(W, s).double()
+    ref = x.double() @ wd.T
+    h = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6) * (1.0 + nw.double())
+    refn = h @ wd.T
+    Wd, sd, xd, nwd = W.to(dev), s.to(dev), x.to(dev), nw.to(dev)
+    announce(f"gemv matrix core M{M} N{N} K{K} gs {gs}")
+    y = ops.gemv(xd, Wd, sd)
+    assert oracle.rel_err(y.cpu(), ref) <= 2e-6
+    yn = ops.gemv(xd, Wd, sd, prenorm=(None, nwd, 1e-6, None))
+    assert oracle.rel_err(yn.cpu(), refn) <= 2e-6
+    base = torch.randn(M, N, generator=g) * float(ref.std())
+    acc = base.to(dev)
+    ops.gemv(xd, Wd, sd, out=acc, epilogue="add")
+    assert oracle.rel_err(acc.cpu(), base.double() + ref) <= 2e-6
+    if N % 2 == 0:
+        pushes = [(3, "add", [1.0, -2.0, 0.5, 4.0]), (1 << 30, "add", [9.0]), (N // 2 - 1, "mul", [0.5, 2.0, 1.0, -1.0])]
+        exp = omlp.swiglu_push(refn[:, 0::2].float(), refn[:, 1::2].float(), pushes, T=1)
+        a = ops.gemv(xd, Wd, sd, epilogue="swiglu", pushes=ops.pack_pushes(pushes, dev), prenorm=(None, nwd, 1e-6, None))
+        assert oracle.rel_err(a.cpu(), exp) <= 5e-6  # (the silu's exp and reciprocal: 1 ulp each)
+
+
+@pytest.mark.parametrize("M,N", [(3, 64), (4, 64), (8, 64), (4, 16400)])
+def test_gemv_infinities_and_nan_stay_in_their_row(M, N):
+    """An infinity or NaN in a row of x reaches that row's outputs as fp32 arithmetic has it (inf times a weight of
+    either sign, inf times zero, NaN; a signalling NaN too) and no other row's; the largest finite value and subnormals
+    do not overflow in the split."""
+    dev = device()
+    g = torch.Generator().manual_seed(M)
+    W = torch.randint(-127, 128, (N, 512), generator=g, dtype=torch.int8)
+    W[5, 7] = 0
+    W[:, 0] = 1  # (the scale is applied to the sum: a larger weight would overflow it in any form)
+    s = torch.rand(N, generator=g) * 0.01
+    x = torch.randn(M, 512, generator=g)
+    x[0, 7] = float("inf")
+    x[1, 300] = float("nan")
+    x.view(torch.int32)[2, 9] = 0x7F800001  # a signalling NaN whose payload is in the low half only
+    clean = M > 3
+    if clean:
+        x[3, 0], x[3, 1] = 3.4028234e38, 1e-40
+    ref = x.double() @ omlp.q8_dequant(W, s).double().T
+    announce(f"gemv nonfinite M{M} N{N}")
+    y = ops.gemv(x.to(dev), W.to(dev), s.to(dev)).cpu()
+    assert bool(y[1].isnan().all()) and bool(y[2].isnan().all())
+    assert bool(y[0, 5].isnan()) and torch.equal(y[0].isinf(), ref[0].isinf())
+    inf = ref[0].isinf()
+    assert torch.equal(y[0][inf].sign().double(), ref[0][inf].sign())
+    for m in range(3, M):
+        ok = ref[m].abs() < 3e38
+        assert bool(y[m][ok].isfinite().all())
+        assert oracle.rel_err(y[m][ok], ref[m][ok]) <= 2e-6
