@@ -329,7 +329,7 @@ struct PfStage {
 // Work items. Query block qb needs key tiles 0 .. nkt(qb) - 1, so the causal blocks range from 1 to ~T/64 tiles. With
 // a split length Ls > 0, every block with more than Ls tiles (qb >= 2 Ls) is run as two items, tiles [0, Ls) and
 // [Ls, nkt), whose (O, m, l) are combined by attn_prefill_merge_kernel; the others run whole (Ls = 0, every block
-// whole and longest first, when the estimate of pf_split_pays finds that faster). Two orders:
+// whole and longest first, when the estimate of pf_schedule finds that faster). Two orders:
 // - Independent items, numbered longest first: all first halves (Ls tiles each), then second halves and whole blocks
 //   alternately, each in decreasing length, so that the hardware's in-order dispatch to free CUs balances the CUs'
 //   total tiles. Used when the items outnumber the CUs.
@@ -389,6 +389,57 @@ inline int pf_items(int nqb, int Ls, bool paired) {
   return paired ? nsq + (nsq > qs ? nsq : qs) : 2 * nsq + qs;
 }
 
+// Key-range splits (KS): the third schedule, for launches whose query blocks leave CUs idle even in halves (a prompt of
+// 1000 tokens on one row: 64 blocks; a 128-token chunk on three rows over the cache: 24). Query block qb of nkt tiles is
+// cut into ceil(nkt / per) runs of per = max(min_per, ceil(nkt / NS)) tiles, one block each, block order s * nqb + (nqb -
+// 1 - qb); blocks past a query block's runs exit, and a query block of one run writes its output itself. A run must not
+// start past the block's first query (its lanes' running max would stay -inf), so starts are clipped to `full`, the
+// tiles entirely at or below that query; nkt is at most full + 2 and per at least kKsMinTiles, so no run is empty.
+// What bounds those launches is one block's chain of tiles (about 2.1 us each) with most CUs idle. Measured on MI355X, 8
+// query / 2 kv heads, us, key runs against the better of the other schedules: own keys, one row of 500 / 1000 / 2000 /
+// 2500 tokens 31.5 / 41.2 / 54.2 / 67.3 against 41.8 / 52.3 / 70.2 / 80.2, two rows of 1000 44.8 / 54.5, three rows of
+// 1000 51.5 / 58.7; over the cache (front end included), 2 tokens at 1700 keys 26.3 / 63.8, at 7000 39.7 / 217; three rows
+// of 128 tokens at 1700 keys 40.2 / 77.0. Runs of at least 4 tiles: a partial and its share of the merge cost about half
+// a tile. A cache of under 12 tiles is not cut (5 tiles as 4 + 1: 30.9 against 27.9); a short context in a longer cache
+// pays the merge's launch, 1.7 us of 20-30, since its length is on the device.
+constexpr int kKsMinTiles = 4;
+
+struct PfRun {
+  int kt0, kt1, n;  // tiles of run s, number of runs
+};
+
+__host__ __device__ inline PfRun pf_run(int nkt, int full, int min_per, int NS, int s) {
+  const int even = (nkt + NS - 1) / NS, per = even > min_per ? even : min_per;
+  const int n = (nkt + per - 1) / per;
+  const int a = s * per, e = a + per;
+  return {a < full ? a : full, s + 1 < n ? (e < full ? e : full) : nkt, n};
+}
+
+// tiles of query block qb: own keys, or over the cache (its first query at position qshift + q0)
+__device__ inline int pf_nkt(bool cached, int qb, int qshift, int T) {
+  return cached ? (qshift + min(qb * kBQ + kBQ - 1, T - 1)) / kBN + 1 : pf_tiles(qb);
+}
+
+// The own-keys form's run length: the shortest whose runs fit `slots` blocks at once; 0: none, or one run per block.
+// *ns: the most runs of a block.
+inline int pf_ks_len(int nqb, int64_t n_other, int slots, int* ns) {
+  if ((int64_t)nqb * n_other >= slots) return 0;
+  const int nmax = pf_tiles(nqb - 1);
+  if (nmax < 2 * kKsMinTiles) return 0;
+  int64_t tiles = 0;
+  for (int qb = 0; qb < nqb; ++qb) tiles += pf_tiles(qb);
+  const int64_t least = (tiles * n_other + slots - 1) / slots;
+  for (int per = least > kKsMinTiles ? (int)least : kKsMinTiles; per < nmax; ++per) {
+    int64_t runs = 0;
+    for (int qb = 0; qb < nqb && runs * n_other <= slots; ++qb)
+      runs += (pf_tiles(qb) + per - 1) / per;
+    *ns = (nmax + per - 1) / per;
+    if (runs * n_other <= slots && (int64_t)nqb * n_other * *ns <= 2 * (int64_t)slots) return per;
+  }
+  return 0;
+}
+constexpr int kKsSlots = 256;  // the blocks that the workspace holds runs for (one per CU of the MI355X), twice over
+
 // Estimated end of a launch's blocks (in units of one tile's time) under the hardware's in-order dispatch, each block
 // taken by the CU that frees first (one block per CU at a time). A block costs its tiles, 1.5 for its query prologue
 // and epilogue, and 0.5 more for a split half's partial stores.
@@ -410,56 +461,79 @@ static double pf_dispatch_time(int nqb, int Ls, bool paired, int64_t n_other, in
   return end;
 }
 
-// Whether splitting the long query blocks pays on a device of cus CUs: the split schedule's estimated end plus the
-// merge kernel (1 for its launch, 0.04 per pair of halves of four waves: the partials' stores and reads) against
-// the longest-first order of whole blocks. The costs were fitted to same-box timings of both schedules over ten
-// shapes (B 1-4, T 1536-8192, 8 q / 2 kv heads), whose faster schedule they all pick. Decisions are kept per shape.
-static bool pf_split_pays(int nqb, int Ls, int64_t n_other, int gw, int cus) {
-  if (Ls == 0) return false;
-  if (cus <= 0) return true;
-  const int64_t nsq = nqb - 2 * Ls;
+// The schedule of a launch on a device of cus CUs: 0 whole blocks, longest first; 1 the long blocks in halves (Ls); 2 key
+// runs. Halves: the split schedule's estimated end plus the merge kernel (1 for its launch, 0.04 per pair of halves of
+// four waves: the partials' stores and reads). The costs were fitted to same-box timings of both schedules over ten
+// shapes (B 1-4, T 1536-8192, 8 q / 2 kv heads), whose faster schedule they all pick. Key runs: the longest run, 2 for
+// prologue and partial, and 0.04 per partial of four waves, against 1.25 times the halves' estimate, which is short for the
+// blocks under 40 tiles that have this option (fitted to B 1-3, T 300-2896). Decisions are kept per shape.
+static int pf_schedule(int nqb, int Ls, int ks_per, int64_t n_other, int gw, int cus) {
+  if (Ls == 0 && ks_per == 0) return 0;
+  if (cus <= 0) return Ls ? 1 : 0;
+  const int64_t nsq = Ls ? nqb - 2 * Ls : 0;
   // past 256 K blocks (a simulation of about 10 ms) the whole blocks spread evenly however long the longest is
-  if ((int64_t)pf_items(nqb, Ls, false) * n_other > ((int64_t)1 << 18)) return false;
+  if ((int64_t)pf_items(nqb, Ls, false) * n_other > ((int64_t)1 << 18)) return 0;
   struct Key {
     int nqb, gw, cus;
     int64_t n_other;
   };
   static std::mutex mu;
   static Key keys[32];
-  static bool vals[32];
+  static int vals[32];
   static int nkeys = 0, next = 0;
   {
     std::lock_guard<std::mutex> lock(mu);
     for (int i = 0; i < nkeys; ++i)
       if (keys[i].nqb == nqb && keys[i].gw == gw && keys[i].cus == cus && keys[i].n_other == n_other) return vals[i];
   }
-  const bool paired = (int64_t)pf_items(nqb, Ls, true) * n_other <= cus;
-  const double split = pf_dispatch_time(nqb, Ls, paired, n_other, cus) + 1.0 + 0.01 * gw * (double)(nsq * n_other);
-  const bool pays = split < pf_dispatch_time(nqb, 0, false, n_other, cus);
+  double best = pf_dispatch_time(nqb, 0, false, n_other, cus);
+  int pick = 0;
+  if (Ls) {
+    const bool paired = (int64_t)pf_items(nqb, Ls, true) * n_other <= cus;
+    const double split = pf_dispatch_time(nqb, Ls, paired, n_other, cus) + 1.0 + 0.01 * gw * (double)(nsq * n_other);
+    if (split < best) {
+      best = split;
+      pick = 1;
+    }
+  }
+  if (ks_per && cus >= kKsSlots) {
+    if (pick == 1) best *= 1.25;
+    int64_t parts = 0;
+    for (int qb = 0; qb < nqb; ++qb) {
+      const int n = (pf_tiles(qb) + ks_per - 1) / ks_per;
+      parts += n > 1 ? n : 0;
+    }
+    if (ks_per + 2.0 + 0.01 * gw * (double)(parts * n_other) < best) pick = 2;
+  }
   std::lock_guard<std::mutex> lock(mu);
   keys[next] = Key{nqb, gw, cus, n_other};
-  vals[next] = pays;
+  vals[next] = pick;
   next = (next + 1) % 32;
   nkeys = nkeys < 32 ? nkeys + 1 : 32;
-  return pays;
+  return pick;
 }
 
 // GF: the gate is read from the fused projection output (fp32 rows of stride gate_ld, query head h at 2 D h) instead
 // of a [B, T, Hq, D] bf16 tensor.
-template <int GW, bool PAIRED, bool GF>
+// KS: key runs; Ls is then the shortest run and NS the most runs of a query block.
+template <int GW, bool PAIRED, bool GF, bool KS>
 __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kr, const __bf16* __restrict__ vt,
     const void* __restrict__ gate, int64_t gate_ld, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     int pos0, __bf16* __restrict__ out, int T, int Tp, int Hq, int Hkv, int ngroups, int rot, float scale, int nqb,
-    int B, int Ls, float* __restrict__ part, const int32_t* __restrict__ pos_dev) {
+    int B, int Ls, int NS, float* __restrict__ part, const int32_t* __restrict__ pos_dev) {
   Q35_ARGS_UPFRONT(q, kr, vt, gate, gate_ld, cos_t, sin_t, pos0, out, T, Tp, Hq, Hkv, ngroups, rot, scale, nqb, B, Ls,
-                   part, pos_dev);
+                   NS, part, pos_dev);
+  static_assert(!(PAIRED && KS), "one schedule");
   __shared__ PfStage stage[2];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_other = B * Hkv * ngroups;
-  const PfItem it0 = pf_item((int)(blockIdx.x / n_other), nqb, Ls, PAIRED);
+  const int item = (int)(blockIdx.x / n_other);
+  PfItem it0;
+  if constexpr (KS) it0 = PfItem{nqb - 1 - item % nqb, 0, 0, item / nqb, -1};
+  else it0 = pf_item(item, nqb, Ls, PAIRED);
   const int rem = blockIdx.x % n_other;
   const int b = rem / (Hkv * ngroups);
   const int kvh = (rem / ngroups) % Hkv;
@@ -515,8 +589,15 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
   auto run = [&](PfItem it) {
     const int qb = it.qb;
     const int q0 = qb * kBQ;
-    // cached mode: the block's key tiles end at its last query's position
-    if (pos_dev) it.kt1 = (qshift + min(q0 + kBQ - 1, T - 1)) / kBN + 1;
+    if constexpr (KS) {
+      const PfRun r = pf_run(pf_nkt(pos_dev != nullptr, qb, qshift, T), (qshift + q0) / kBN, Ls, NS, it.half);
+      if (it.half >= r.n) return;
+      it.kt0 = r.kt0;
+      it.kt1 = r.kt1;
+      if (r.n == 1) it.half = -1;
+    } else if (pos_dev) {  // cached mode: the block's key tiles end at its last query's position
+      it.kt1 = pf_nkt(true, qb, qshift, T);
+    }
 
     // ---- Q^T operand (B of S^T = K Q^T): lane holds query q0 + ln, dims 16 ks + 8 hh + j, rotated. Every load (the
     //      query row, the rotation partners and the cos / sin rows) is issued before the first tile's copies and before
@@ -741,8 +822,9 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
 
     // ---- a split query block: each half publishes its (O, m, l); attn_prefill_merge_kernel combines them ----
     if (it.half >= 0) {
-      const int pair = (qb - 2 * Ls) * n_other + rem;
-      float* mine = part + ((size_t)(2 * pair + it.half) * GW + wave) * kPartFloats;
+      const size_t slot = KS ? ((size_t)qb * n_other + rem) * NS + it.half
+                             : 2 * (size_t)((qb - 2 * Ls) * n_other + rem) + it.half;
+      float* mine = part + (slot * GW + wave) * kPartFloats;
 #pragma unroll
       for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
@@ -907,6 +989,91 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
   }
 }
 
+// Kernel 3 of the key-run schedule: the runs of a query block, combined in run order, as above. One block per (query
+// block and (row, kv head, group), query head of the group); query blocks of one run have nothing to merge.
+template <int GW, bool GF>
+__global__ __launch_bounds__(256) void attn_prefill_merge_runs_kernel(const float* __restrict__ part,
+                                                                      const void* __restrict__ gate, int64_t gate_ld,
+                                                                      __bf16* __restrict__ out, int T, int Tp, int Hq,
+                                                                      int Hkv, int ngroups, int B, int min_per, int NS,
+                                                                      const int32_t* __restrict__ pos_dev) {
+  Q35_ARGS_UPFRONT(part, gate, gate_ld, out, T, Tp, Hq, Hkv, ngroups, B, min_per, NS, pos_dev);
+  const int pair = blockIdx.x, wave = blockIdx.y, tid = threadIdx.x;
+  const int n_other = B * Hkv * ngroups;
+  const int qb = pair / n_other, rem = pair % n_other;
+  const int b = rem / (Hkv * ngroups), kvh = (rem / ngroups) % Hkv, hg = rem % ngroups;
+  const int h = kvh * (Hq / Hkv) + hg * GW + wave;
+  const int qshift = pos_dev ? min(max(pos_dev[b], 0), Tp - T) : 0;
+  const int n = pf_run(pf_nkt(pos_dev != nullptr, qb, qshift, T), (qshift + qb * kBQ) / kBN, min_per, NS, 0).n;
+  if (n == 1) return;
+  const int l = tid & 63, tq = qb * kBQ + (l & 31);  // every chunk of thread t has lane l = t & 63
+  const float* p0 = part + ((size_t)pair * NS * GW + wave) * kPartFloats;
+  const size_t run = (size_t)GW * kPartFloats;
+  f32x4 gf[8];
+  u32x2 gr[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int mtc = (tid + 256 * j) >> 6, d = 8 * mtc + 4 * (l >> 5), tr = min(tq, T - 1);
+    if constexpr (GF)
+      gf[j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(gate) + ((size_t)b * T + tr) * gate_ld +
+                                              (size_t)h * 2 * kPD + d);
+    else
+      gr[j] = *reinterpret_cast<const u32x2*>(static_cast<const __bf16*>(gate) +
+                                              ((size_t)b * T + tr) * (size_t)Hq * kPD + (size_t)h * kPD + d);
+  }
+  // the running (O, m, l) over the runs, rescaled as the maximum moves; the next run's loads go out first
+  f32x4 o[8], w[2][8];
+  float mw[2], lw[2];
+  auto load = [&](int r, int i) {
+    const float* p = p0 + r * run;
+    mw[i] = p[8192 + l];
+    lw[i] = p[8192 + 64 + l];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[i][j] = *reinterpret_cast<const f32x4*>(p + (size_t)(tid + 256 * j) * 4);
+  };
+  float mm = -INFINITY, lt = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = zero4();
+  auto add = [&](int i) {  // (every run's maximum is finite)
+    const float mn = fmaxf(mm, mw[i]);
+    const float c0 = __builtin_amdgcn_exp2f(mm - mn), c1 = __builtin_amdgcn_exp2f(mw[i] - mn);
+    mm = mn;
+    lt = fmaf(lt, c0, lw[i] * c1);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[j][q] = fmaf(o[j][q], c0, w[i][j][q] * c1);
+  };
+  load(0, 0);
+  for (int r = 0; r < n; r += 2) {
+    load(min(r + 1, n - 1), 1);
+    add(0);
+    if (r + 1 == n) break;
+    load(min(r + 2, n - 1), 0);
+    add(1);
+  }
+  if (tq >= T) return;
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int mtc = (tid + 256 * j) >> 6, d = 8 * mtc + 4 * (l >> 5);
+    float gv[4];
+    if constexpr (GF) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) gv[q] = gf[j][q];
+    } else {
+      gv[0] = bf16lo(gr[j][0]);
+      gv[1] = bf16hi(gr[j][0]);
+      gv[2] = bf16lo(gr[j][1]);
+      gv[3] = bf16hi(gr[j][1]);
+    }
+    bf16x4 ov;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ov[q] = (__bf16)(o[j][q] * inv * sigmoidf_(gv[q]));
+    *reinterpret_cast<bf16x4*>(out + ((size_t)b * T + tq) * (size_t)Hq * kPD + (size_t)h * kPD + d) = ov;
+  }
+}
+
 static int64_t padded_T(int64_t T) { return (T + kBN - 1) / kBN * kBN; }
 
 // Compute units of the current device, queried once per device (the paired work order needs every block resident).
@@ -923,10 +1090,12 @@ static int device_cus() {
 }
 
 // Workspace: K rotated and V transposed ([B, Hkv, Tp, D] bf16 each), for the projection-output form the rotated
-// queries ([B, T, Hq, D] bf16), then the split blocks' partials ([pairs][2 halves][wave] x kPartFloats fp32).
+// queries ([B, T, Hq, D] bf16), then the partials of the split blocks ([pairs][2 halves][wave] x kPartFloats fp32) or of the
+// key runs ([query block and (row, kv head, group)][NS runs][wave]).
 struct PfLayout {
   size_t q_off, part_off, total;
   int64_t npairs;
+  int ks_per, ks_ns;  // key runs: the shortest run, the most runs of a query block (0: not an option)
 };
 // Ls: the split length (the workspace functions size for pf_split_len, the most a launch can use).
 static PfLayout pf_layout(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, bool fp, int Ls) {
@@ -939,7 +1108,11 @@ static PfLayout pf_layout(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, bool fp
   l.npairs = nsq * B * Hkv * (G / GW);
   l.q_off = (size_t)2 * B * Hkv * Tp * kPD * sizeof(__bf16);
   l.part_off = l.q_off + (fp ? ((size_t)B * T * Hq * kPD * sizeof(__bf16) + 255) / 256 * 256 : 0);
-  l.total = (l.part_off + (size_t)2 * l.npairs * GW * kPartFloats * sizeof(float) + 255) / 256 * 256;
+  int ns = 0;
+  l.ks_per = pf_ks_len((int)nqb, B * Hkv * (G / GW), kKsSlots, &ns);
+  l.ks_ns = l.ks_per ? ns : 0;
+  const size_t runs = (size_t)l.ks_ns * nqb * B * Hkv * (G / GW), halves = (size_t)2 * l.npairs;
+  l.total = (l.part_off + (runs > halves ? runs : halves) * GW * kPartFloats * sizeof(float) + 255) / 256 * 256;
   return l;
 }
 
@@ -978,10 +1151,13 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
     return Q35_EWORKSPACE;
   // the first HIP call: the device's compute units decide the split and the work order
   const int cus = device_cus();
-  const int Ls = pf_split_pays((int)nqb, Lmax, n_other, GW, cus) ? Lmax : 0;
+  const PfLayout lay0 = pf_layout(B, T, Hq, Hkv, FP, Lmax);
+  const int sched = pf_schedule((int)nqb, Lmax, lay0.ks_per, n_other, GW, cus);
+  const bool runs = sched == 2;
+  const int Ls = sched == 1 ? Lmax : 0;
   const PfLayout lay = pf_layout(B, T, Hq, Hkv, FP, Ls);
   const bool paired = Ls > 0 && (int64_t)pf_items((int)nqb, Ls, true) * n_other <= cus;
-  const int64_t nblocks = (int64_t)pf_items((int)nqb, Ls, paired) * n_other;
+  const int64_t nblocks = runs ? (int64_t)nqb * lay.ks_ns * n_other : (int64_t)pf_items((int)nqb, Ls, paired) * n_other;
   char* ws = static_cast<char*>(workspace);
   __bf16* kr = reinterpret_cast<__bf16*>(ws);
   __bf16* vt = kr + (size_t)B * Hkv * Tp * kPD;
@@ -1006,11 +1182,16 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
   // the projection-output form's queries are rotated by the pre-pass: the main kernel then rotates nothing
   const int mrot = FP ? 0 : (int)rot;
 #define Q35_PF_LAUNCH(GG)                                                                                           \
-  hipLaunchKernelGGL((paired ? attn_prefill_kernel<GG, true, FP> : attn_prefill_kernel<GG, false, FP>),            \
+  hipLaunchKernelGGL((runs ? attn_prefill_kernel<GG, false, FP, true>                                               \
+                           : paired ? attn_prefill_kernel<GG, true, FP, false> : attn_prefill_kernel<GG, false, FP, false>), \
                      dim3((unsigned)nblocks), dim3(64 * GG), 0, st, (const __bf16*)q, kr, vt, gate, gate_ld, cos, sin, \
                      (int)pos0, (__bf16*)out, (int)T, (int)Tp, (int)Hq, (int)Hkv, ngroups, mrot, scale, (int)nqb,     \
-                     (int)B, Ls, part, (const int32_t*)nullptr);                                                    \
-  if (lay.npairs > 0)                                                                                               \
+                     (int)B, runs ? lay.ks_per : Ls, lay.ks_ns, part, (const int32_t*)nullptr);                     \
+  if (runs)                                                                                                         \
+    hipLaunchKernelGGL((attn_prefill_merge_runs_kernel<GG, FP>), dim3((unsigned)(nqb * n_other), GG), dim3(256), 0, st, \
+                       part, gate, gate_ld, (__bf16*)out, (int)T, (int)Tp, (int)Hq, (int)Hkv, ngroups, (int)B,       \
+                       lay.ks_per, lay.ks_ns, (const int32_t*)nullptr);                                             \
+  else if (lay.npairs > 0)                                                                                          \
     hipLaunchKernelGGL((attn_prefill_merge_kernel<GG, FP>), dim3((unsigned)lay.npairs, GG), dim3(256), 0, st, part,  \
                        gate, gate_ld, (__bf16*)out, (int)T, (int)Hq, (int)Hkv, ngroups, (int)B, Ls)
   switch (GW) {
@@ -1106,9 +1287,9 @@ extern "C" int q35_gated_attn_prefill_cached(const void* q, const void* k_cache,
                      0, st, (const __bf16*)v_cache, pos, vt, (int)T, (int)max_len, (int)Hkv);
   // one item per query block (no key split: the key range depends on the device positions), latest block first
 #define Q35_PFC_LAUNCH(GG)                                                                                        \
-  hipLaunchKernelGGL((attn_prefill_kernel<GG, false, false>), dim3((unsigned)nblocks), dim3(64 * GG), 0, st,     \
+  hipLaunchKernelGGL((attn_prefill_kernel<GG, false, false, false>), dim3((unsigned)nblocks), dim3(64 * GG), 0, st,     \
                      (const __bf16*)q, (const __bf16*)k_cache, vt, gate, Hq * kPD, cos, sin, 0, (__bf16*)out,      \
-                     (int)T, (int)max_len, (int)Hq, (int)Hkv, ngroups, (int)rot, scale, (int)nqb, (int)B, 0,        \
+                     (int)T, (int)max_len, (int)Hq, (int)Hkv, ngroups, (int)rot, scale, (int)nqb, (int)B, 0, 0,     \
                      (float*)nullptr, pos)
   switch (GW) {
     case 1: Q35_PFC_LAUNCH(1); break;
@@ -1124,6 +1305,19 @@ extern "C" int q35_gated_attn_prefill_cached(const void* q, const void* k_cache,
 static size_t pfc_proj_q_off(int64_t B, int64_t Hkv, int64_t max_len) {
   return ((size_t)B * Hkv * q35::kPD * max_len * sizeof(__bf16) + 255) / 256 * 256;
 }
+static size_t pfc_proj_part_off(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t max_len) {
+  return pfc_proj_q_off(B, Hkv, max_len) + ((size_t)B * T * Hq * q35::kPD * sizeof(__bf16) + 255) / 256 * 256;
+}
+// The most key runs of a query block over the cache (its length is known on the device only): as many as fill the device
+// once, of at least kKsMinTiles tiles of the whole cache; 1: no split.
+static int pfc_runs(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t max_len) {
+  using namespace q35;
+  const int64_t G = Hq / Hkv, GW = G > 4 ? 4 : G;
+  const int64_t blocks = (T + kBQ - 1) / kBQ * B * Hkv * (G / GW);
+  const int64_t fit = kKsSlots / blocks, most = max_len / kBN / kKsMinTiles;
+  const int64_t n = most < 3 ? 1 : fit < most ? fit : most;
+  return n < 1 ? 1 : n > 16 ? 16 : (int)n;
+}
 
 extern "C" size_t q35_gated_attn_prefill_cached_proj_workspace_bytes(int64_t B, int64_t T, int64_t Hq, int64_t Hkv,
                                                                      int64_t D, int64_t max_len) {
@@ -1134,7 +1328,9 @@ extern "C" size_t q35_gated_attn_prefill_cached_proj_workspace_bytes(int64_t B, 
   const int64_t G = Hq / Hkv;
   if (G != 1 && G != 2 && G != 4 && G != 8) return 0;
   if (max_len > ((int64_t)1 << 30) || B * Hq > ((int64_t)1 << 30)) return 0;
-  return pfc_proj_q_off(B, Hkv, max_len) + ((size_t)B * T * Hq * kPD * sizeof(__bf16) + 255) / 256 * 256;
+  const int64_t GW = G > 4 ? 4 : G, runs = pfc_runs(B, T, Hq, Hkv, max_len);
+  const size_t parts = runs > 1 ? (size_t)runs * ((T + kBQ - 1) / kBQ) * B * Hkv * (G / GW) : 0;
+  return (pfc_proj_part_off(B, T, Hq, Hkv, max_len) + parts * GW * kPartFloats * sizeof(float) + 255) / 256 * 256;
 }
 
 extern "C" int q35_gated_attn_prefill_cached_proj(const float* y, int64_t ldy, const float* q_norm_w,
@@ -1184,11 +1380,19 @@ extern "C" int q35_gated_attn_prefill_cached_proj(const float* y, int64_t ldy, c
   }
 #undef Q35_KVC_LAUNCH
   // the queries arrive rotated (rot 0 in the main kernel); keys from the cache, the gate from y
+  const int runs = pfc_runs(B, T, Hq, Hkv, max_len);
+  float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + pfc_proj_part_off(B, T, Hq, Hkv, max_len));
 #define Q35_PFCP_LAUNCH(GG)                                                                                        \
-  hipLaunchKernelGGL((attn_prefill_kernel<GG, false, true>), dim3((unsigned)nblocks), dim3(64 * GG), 0, st,        \
-                     (const __bf16*)qr, (const __bf16*)k_cache, vt, (const void*)(y + kPD), ldy, cos, sin, 0,      \
-                     (__bf16*)out, (int)T, (int)max_len, (int)Hq, (int)Hkv, ngroups, 0, scale, (int)nqb, (int)B, 0, \
-                     (float*)nullptr, pos)
+  hipLaunchKernelGGL((runs > 1 ? attn_prefill_kernel<GG, false, true, true>                                        \
+                               : attn_prefill_kernel<GG, false, true, false>),                                     \
+                     dim3((unsigned)(nblocks * runs)), dim3(64 * GG), 0, st, (const __bf16*)qr,                    \
+                     (const __bf16*)k_cache, vt, (const void*)(y + kPD), ldy, cos, sin, 0, (__bf16*)out, (int)T,   \
+                     (int)max_len, (int)Hq, (int)Hkv, ngroups, 0, scale, (int)nqb, (int)B,                         \
+                     runs > 1 ? kKsMinTiles : 0, runs, part, pos);                                                 \
+  if (runs > 1)                                                                                                    \
+    hipLaunchKernelGGL((attn_prefill_merge_runs_kernel<GG, true>), dim3((unsigned)nblocks, GG), dim3(256), 0, st,   \
+                       part, (const void*)(y + kPD), ldy, (__bf16*)out, (int)T, (int)max_len, (int)Hq, (int)Hkv,    \
+                       ngroups, (int)B, kKsMinTiles, runs, pos)
   switch (GW) {
     case 1: Q35_PFCP_LAUNCH(1); break;
     case 2: Q35_PFCP_LAUNCH(2); break;

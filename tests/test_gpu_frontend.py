@@ -234,7 +234,11 @@ def test_attn_prefill_from_projection(B, T, Hq, Hkv, pos0, max_len):
 # Rows at different positions (0, mid-cache, the last rows), ragged key ranges, GQA 1 / 4 / 8, one token.
 @pytest.mark.parametrize("B,T,Hq,Hkv,max_len,pos", [(3, 100, 8, 2, 448, [0, 37, 300]), (2, 1, 8, 2, 256, [5, 255]),
                                                      (1, 257, 4, 4, 640, [383]), (2, 64, 8, 1, 192, [128, 0]),
-                                                     (1, 130, 16, 2, 320, [64])])
+                                                     (1, 130, 16, 2, 320, [64]),
+                                                     # long caches: key runs, on rows of one run and of many, runs that
+                                                     # end on the call's first tile, GQA 8 (two groups) and 1
+                                                     (3, 100, 8, 2, 2304, [0, 1000, 2204]), (1, 2, 8, 2, 1024, [63]),
+                                                     (2, 33, 16, 2, 1024, [64, 991]), (1, 128, 4, 4, 768, [640])])
 def test_attn_prefill_over_cache_from_projection(B, T, Hq, Hkv, max_len, pos):
     """The multi-token call over the cache from the fused projection output (q35_gated_attn_prefill_cached_proj: the
     front end and the cache append in the pre-pass, whose value blocks take the earlier rows from the cache and the
@@ -272,6 +276,8 @@ def test_attn_prefill_over_cache_from_projection(B, T, Hq, Hkv, max_len, pos):
     e_ref, e_two = oracle.rel_err(out.float().cpu(), ref), oracle.rel_err(out.float().cpu(), two.float().cpu())
     print(f"prefill over cache from projection: rel err {e_ref:.3e} (oracle), {e_two:.3e} (two-launch path)")
     assert out.shape == (B, T, Hq * D) and e_ref <= 2e-2 and e_two <= 1e-2
+    rows = (out.float().cpu() - ref).norm(dim=-1) / ref.norm(dim=-1)  # each query row by itself
+    assert float(rows.max()) <= 3e-2
 
 
 @pytest.mark.parametrize("with_add", [False, True])
