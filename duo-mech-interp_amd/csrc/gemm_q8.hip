@@ -28,7 +28,7 @@
 //     (so that stage s's buffer is free at the next barrier). The tiles of one XCD are consecutive (n fastest inside
 //     an m panel), so a panel's x stays in that XCD's L2. LDS rows are XOR-swizzled so that the 16-byte accesses of
 //     16 consecutive lanes hit distinct banks. The SwiGLU epilogue splits each (gate, up) lane pair's rows between
-//     the two lanes.
+//     the two lanes and turns the activations into whole rows in LDS.
 //   gemm_q8_rs_kernel (the rest: the N = 1024 output and down projections): 2 x 2 waves over BM x 128 tiles, x and W
 //     staged through registers into LDS (split and widened on the way), the next K step's loads issued before the
 //     current step's MFMAs; two blocks per CU.
@@ -364,8 +364,71 @@ __global__ __launch_bounds__(512, 1) void gemm_q8_dma_kernel(const float* __rest
   }
 
   // epilogue: lane holds column n = n0 + 64 wn + 32 nt + l32, rows m0 + 64 wm + 32 mt + 8 (r / 4) + 4 lh + r % 4
+  if constexpr (EPI == kGemmSwiglu) {
+    // Activations through LDS, so that they leave as whole rows: straight from the accumulators, a store instruction
+    // held 16 neurons of four rows, in the split layout as single bf16 values (gate/up at 6144 rows, split output, under the
+    // profiler: 302 us, through 64 KB of the free stages 258). Columns n (gate, even lane) and n + 1 (up, odd lane) of a neuron: the even
+    // lane finishes the rows with r < 8, the odd lane those with r >= 8. Row r of the tile lies at 128 r with neuron c at
+    // c ^ 16 ((r / 4) % 2) ^ 32 ((r / 16) % 2): the four rows of one write fall in distinct banks.
+    const bool pushes_here = gemm_pushes_touch(pushes, npush, n0 >> 1, (n0 + kDBN) >> 1);
+    float* const act = reinterpret_cast<float*>(smem);
+    auto at = [](int r, int c) { return 128 * r + (c ^ (((r >> 2) & 1) << 4) ^ (((r >> 4) & 1) << 5)); };
+    const bool odd = (l32 & 1) != 0;
+    lds_barrier();  // every wave has read its last fragments
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = n0 + wn * 64 + 32 * nt + l32, neuron = n >> 1;
+      const float sc = GS ? 1.f : ws[min(n, N - 1)];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float v0 = acc[mt][nt][i] * sc, v1 = acc[mt][nt][i + 8] * sc;
+          const float o = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? v0 : v1), 0xB1, 0xF, 0xF, false));
+          float a = gemm_silu(odd ? o : v0) * (odd ? v1 : o);
+          const int row = wm * 64 + 32 * mt + 8 * (i >> 2) + (i & 3) + 4 * lh + 16 * (int)odd;
+          if (pushes_here) {
+            const int prow = gemm_push_row(moff + m0 + row, T);
+            for (int p = 0; p < npush; ++p) a = gemm_push(pushes + p, neuron, prow, a);
+          }
+          act[at(row, wn * 32 + 16 * nt + (l32 >> 1))] = a;
+        }
+    }
+    lds_barrier();
+    const int I = N >> 1;
+    const bool vec = (ldy & 3) == 0 && ((uintptr_t)Y & 15) == 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {  // four neurons of a row per thread
+      const int row = (tid + 512 * u) >> 5, c = 4 * (tid & 31);
+      const int m = m0 + row, neuron = (n0 >> 1) + c;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(act + at(row, c));
+      if (m >= M || neuron >= I) continue;
+      float* y = Y + (int64_t)m * ldy;
+      if (ys) {  // (I is a multiple of 8)
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bf16_hl t = bf16_split(v[e]);
+          hi[e] = t.hi;
+          lo[e] = t.lo;
+        }
+        __bf16* g = reinterpret_cast<__bf16*>(y + 8 * (neuron >> 3)) + (neuron & 7);
+        *reinterpret_cast<bf16x4*>(g) = hi;
+        *reinterpret_cast<bf16x4*>(g + 8) = lo;
+      } else if (vec && neuron + 4 <= I) {
+        *reinterpret_cast<f32x4*>(y + neuron) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (neuron + e < I) y[neuron + e] = v[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (neuron + e < I) gemm_capture(cap, moff + m, T, neuron + e, v[e]);
+    }
+    return;
+  }
   const int mb = m0 + wm * 64 + 4 * lh;
-  const bool pushes_here = EPI == kGemmSwiglu && gemm_pushes_touch(pushes, npush, n0 >> 1, (n0 + kDBN) >> 1);
   int64_t roff[16];  // element offsets of a tile's 16 accumulator rows from its first (uniform): one add per output
 #pragma unroll
   for (int r = 0; r < 16; ++r) roff[r] = (int64_t)(8 * (r >> 2) + (r & 3)) * ldy;
@@ -375,29 +438,12 @@ __global__ __launch_bounds__(512, 1) void gemm_q8_dma_kernel(const float* __rest
     const float sc = GS ? 1.f : ws[min(n, N - 1)];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      float* yt = Y + (int64_t)(mb + 32 * mt) * ldy;
-      float* ytn = yt + (EPI == kGemmSwiglu ? gemm_act_col(n >> 1, ys) : n);
+      float* ytn = Y + (int64_t)(mb + 32 * mt) * ldy + n;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = mb + 32 * mt + 8 * (r >> 2) + (r & 3);
         const float v = acc[mt][nt][r] * sc;
-        if (EPI == kGemmSwiglu) {
-          // columns n (gate, even lane) and n + 1 (up, odd lane) of a neuron: the even lane finishes the rows with
-          // r < 8, the odd lane those with r >= 8
-          const float o = __shfl_xor(v, 1, 64);
-          const bool odd = (l32 & 1) != 0;
-          if (odd == (r >= 8) && m < M && (n | 1) < N) {
-            const int neuron = n >> 1;
-            const float gate = odd ? o : v, up = odd ? v : o;
-            float a = gemm_silu(gate) * up;
-            if (pushes_here) {
-              const int row = gemm_push_row(moff + m, T);
-              for (int p = 0; p < npush; ++p) a = gemm_push(pushes + p, neuron, row, a);
-            }
-            gemm_store_act(ytn + roff[r], neuron, a, ys);
-            gemm_capture(cap, moff + m, T, neuron, a);
-          }
-        } else if (m < M && n < N) {
+        if (m < M && n < N) {
           float* dst = ytn + roff[r];
           *dst = EPI == kGemmAccumulate ? *dst + v : v;
         }
