@@ -27,7 +27,8 @@ def _ptr(t):
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the handle of t's device's current stream, without a Stream object around it (0.1 us against 2.0 a call)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _require(cond, msg):
@@ -40,10 +41,15 @@ def _on_gpu(*ts):
     for t in ts:
         if t is None:
             continue
-        _require(t.is_cuda, "inputs must be HIP device tensors (there is no CPU fallback)")
-        _require(t.is_contiguous(), "inputs must be contiguous")
-        dev = t.device if dev is None else dev
-        _require(t.device == dev, "inputs must be on one device")
+        if not t.is_cuda:
+            raise Q35Error("q35hip: inputs must be HIP device tensors (there is no CPU fallback)")
+        if not t.is_contiguous():
+            raise Q35Error("q35hip: inputs must be contiguous")
+        d = t.get_device()
+        if dev is None:
+            dev = d
+        elif d != dev:
+            raise Q35Error("q35hip: inputs must be on one device")
 
 
 def _workspace(nbytes, device):
@@ -162,7 +168,8 @@ def _gdn_chunk_impl(q, k, v, g, beta, initial_state, chunk_size, scale, use_qk_l
 def _tables_check(cos, sin, rows_needed):
     _require(cos.dtype == torch.float32 and sin.dtype == torch.float32, "cos/sin tables must be fp32")
     _require(cos.dim() == 2 and sin.shape == cos.shape, "cos/sin tables: [P, rot/2]")
-    _require(cos.shape[0] >= rows_needed or cos.shape[1] == 0, f"cos/sin tables need {rows_needed} rows")
+    if cos.shape[0] < rows_needed and cos.shape[1] != 0:
+        raise Q35Error(f"q35hip: cos/sin tables need {rows_needed} rows")
     return 2 * cos.shape[1]
 
 
