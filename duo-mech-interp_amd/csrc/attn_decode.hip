@@ -336,7 +336,7 @@ __global__ __launch_bounds__(256) void attn_decode_partial_kernel(
 #pragma unroll
   for (int hh = 0; hh < G; ++hh)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[hh][e] += __shfl_xor(acc[hh][e], 32, 64);
+    for (int e = 0; e < 8; ++e) acc[hh][e] = add_xor<32>(acc[hh][e]);
   if (lane < 32) {
 #pragma unroll
     for (int hh = 0; hh < G; ++hh)

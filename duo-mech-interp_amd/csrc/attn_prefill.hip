@@ -236,8 +236,7 @@ __global__ __launch_bounds__(256) void attn_kv_prep_kernel(const __bf16* __restr
         const float s1[4] = {p[0] + p[4], p[1] + p[5], p[2] + p[6], p[3] + p[7]};
         const float s2[2] = {s1[0] + s1[2], s1[1] + s1[3]};
         s3[h2] = s2[0] + s2[1];
-        s3[h2] += __shfl_xor(s3[h2], 2, 64);
-        s3[h2] += __shfl_xor(s3[h2], 1, 64);
+        s3[h2] = add_xor<1>(add_xor<2>(s3[h2]));
       }
       rr = rsqrtf((s3[0] + s3[1]) * (1.f / kPD) + fe.eps);
     }
@@ -745,7 +744,7 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
             mx = fmaxf(mx, sc[ksub][i]);
           }
       }
-      return fmaxf(mx, __shfl_xor(mx, 32, 64)) * csc;
+      return max_xor32(mx) * csc;
     };
     // P = 2^(s c - m_run) of tile kt into the row sum, then O^T += V^T P^T: rows = 256 dims (8 tiles of 32), k = 64
     // keys (4 steps of 16). The MFMAs run K step by K step, so those of step kk need only P's group kk: the
@@ -772,7 +771,7 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
           ps += p;
           pb[2 * ksub + (i >> 3)][i & 7] = (__bf16)p;
         }
-      ps += __shfl_xor(ps, 32, 64);
+      ps = add_xor<32>(ps);
       l_run += ps;
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {

@@ -285,12 +285,9 @@ __global__ __launch_bounds__(1024) void gdn_decode_fused_kernel(
     c[e] = s[0][e] * qr[0] + s[1][e] * qr[1] + s[2][e] * qr[2] + s[3][e] * qr[3];
   }
 #pragma unroll
-  for (int off = 8; off < 64; off <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      a[e] += __shfl_xor(a[e], off, 64);
-      c[e] += __shfl_xor(c[e], off, 64);
-    }
+  for (int e = 0; e < 4; ++e) {
+    a[e] = add_xor<32>(add_xor<16>(add_xor<8>(a[e])));
+    c[e] = add_xor<32>(add_xor<16>(add_xor<8>(c[e])));
   }
   if (lane < 8) {
     red[wave][lane][0] = a;
@@ -395,12 +392,9 @@ __global__ __launch_bounds__(256) void gdn_decode_sliced_kernel(
     c[e] = s[0][e] * qr[0] + s[1][e] * qr[1] + s[2][e] * qr[2] + s[3][e] * qr[3];
   }
 #pragma unroll
-  for (int off = 8; off < 64; off <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      a[e] += __shfl_xor(a[e], off, 64);
-      c[e] += __shfl_xor(c[e], off, 64);
-    }
+  for (int e = 0; e < 4; ++e) {
+    a[e] = add_xor<32>(add_xor<16>(add_xor<8>(a[e])));
+    c[e] = add_xor<32>(add_xor<16>(add_xor<8>(c[e])));
   }
   if (lane < 8) {
     red[wave][lane][0] = a;
@@ -510,8 +504,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm4_kernel(const T* __restrict
     for (int e = 0; e < 4; ++e) x[e] = (float)t[e];
   }
   float ss = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
-#pragma unroll
-  for (int off = 1; off < 32; off <<= 1) ss += __shfl_xor(ss, off, 64);
+  ss = add_xor<16>(add_xor<8>(add_xor4_quads(add_xor<2>(add_xor<1>(ss)))));
   const float r = rsqrtf(ss * (1.f / 128.f) + eps);
   const f32x4 zz = *reinterpret_cast<const f32x4*>(z + m * ldz + h * 128 + 4 * hl);
   const f32x4 ww = *reinterpret_cast<const f32x4*>(w + 4 * hl);

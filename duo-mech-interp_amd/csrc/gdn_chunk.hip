@@ -378,8 +378,7 @@ __global__ __launch_bounds__(256, 2) void gdn_pair_prep4_kernel(const __bf16* __
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) ss[i] += __shfl_xor(ss[i], off, 64);
+      ss[i] = add_xor<8>(add_xor4_quads(add_xor<2>(add_xor<1>(ss[i]))));
     }
     if (uc == 0) {
 #pragma unroll
@@ -397,8 +396,7 @@ __global__ __launch_bounds__(256, 2) void gdn_pair_prep4_kernel(const __bf16* __
     float ss = 0.f;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) ss += sumsq8(__builtin_bit_cast(u32x4, qf[a][ks]));
-    ss += __shfl_xor(ss, 16, 64);
-    ss += __shfl_xor(ss, 32, 64);
+    ss = add_xor<32>(add_xor<16>(ss));
     if (lg == 0) cf[3][t] = t < nvalid ? (l2norm ? rsqrtf(ss + 1e-6f) : 1.f) * scale : 0.f;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) qf[a][ks] = __builtin_bit_cast(bf16x8, mask8(__builtin_bit_cast(u32x4, qf[a][ks]), t < nvalid));
@@ -1039,10 +1037,8 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_prep_kernel(const float* __res
     for (int j = 0; j < 8; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) { ssk += kk[j][e] * kk[j][e]; ssq += qq[j][e] * qq[j][e]; }
-    ssk += __shfl_xor(ssk, 1, 64);
-    ssk += __shfl_xor(ssk, 2, 64);
-    ssq += __shfl_xor(ssq, 1, 64);
-    ssq += __shfl_xor(ssq, 2, 64);
+    ssk = add_xor<2>(add_xor<1>(ssk));
+    ssq = add_xor<2>(add_xor<1>(ssq));
     if ((tid & 3) == 0) {
       rkn[row] = l2norm ? rsqrtf(ssk + 1e-6f) : 1.f;
       rqn[row] = l2norm ? rsqrtf(ssq + 1e-6f) : 1.f;

@@ -100,12 +100,9 @@ __global__ __launch_bounds__(256) void gdn_recurrent_kernel(const Tin* __restric
       c[e] = s[0][e] * cur.qr[0] + s[1][e] * cur.qr[1] + s[2][e] * cur.qr[2] + s[3][e] * cur.qr[3];
     }
 #pragma unroll
-    for (int off = 8; off < 64; off <<= 1) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        a[e] += __shfl_xor(a[e], off, 64);
-        c[e] += __shfl_xor(c[e], off, 64);
-      }
+    for (int e = 0; e < 4; ++e) {
+      a[e] = add_xor<32>(add_xor<16>(add_xor<8>(a[e])));
+      c[e] = add_xor<32>(add_xor<16>(add_xor<8>(c[e])));
     }
     if (lane < 8) {
       red[par][wave][lane][0] = a;

@@ -57,29 +57,12 @@ __device__ __forceinline__ float apply_push(const q35_push* ps, int n, int row, 
   return ps->mode ? a * v : a + v;
 }
 
-template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
 // sum over the 16 lanes of a DPP row (lanes 16 r .. 16 r + 15), result in every lane of the row
-__device__ __forceinline__ float row16_sum_f(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  return v + dpp_f<0x140>(v);  // row_mirror
-}
+__device__ __forceinline__ float row16_sum_f(float v) { return add_xor<8>(add_xor4_quads(add_xor<2>(add_xor<1>(v)))); }
 
-// sum over 32 lanes (lanes 0 .. 31 or 32 .. 63) and over the wave, in every lane: DPP within rows of 16, one lane exchange
-// or scalar reads across rows (six lane exchanges through LDS took longer than the loads they waited for)
-__device__ __forceinline__ float half_sum_f(float v) {
-  v = row16_sum_f(v);
-  return v + __shfl_xor(v, 16, 64);
-}
-__device__ __forceinline__ float wave_sum_f(float v) {
-  v = row16_sum_f(v);
-  auto at = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
-  return (at(0) + at(16)) + (at(32) + at(48));
-}
+// sum over 32 lanes (lanes 0 .. 31 or 32 .. 63), and over the wave, in every lane
+__device__ __forceinline__ float half_sum_f(float v) { return add_xor<16>(row16_sum_f(v)); }
+__device__ __forceinline__ float wave_sum_f(float v) { return add_xor<32>(half_sum_f(v)); }
 
 // the prologues' operands (GN: nw is the gated norm's weight) and the epilogues'
 struct GemvArgs {

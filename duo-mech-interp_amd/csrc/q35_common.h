@@ -121,11 +121,50 @@ __device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log
 // The "memory" clobber keeps the compiler from moving memory accesses across it.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Sum / max over the 64 lanes of a wave (butterfly; every lane ends with the result).
+// Lane exchanges on the vector ALU: DPP within rows of 16 lanes, the row swaps of gfx950 across rows. __shfl_xor goes
+// through LDS (ds_bpermute), one round trip of the LDS pipe per step of a reduction. The sums are bitwise those of the
+// xor butterflies they replace. Measured: gate/up GEMV at 3 rows 6.2 -> 6.1 us, attention prefill at 4096 tokens (two
+// exchanges per tile) 108.2 -> 107.6, three rows x 48 tokens + 16 decode steps 14.83 -> 14.73 ms.
+template <int CTRL> __device__ __forceinline__ float lane_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+struct lane_pair {
+  float a, b;  // in every lane: the values of the two lanes OFF apart (in either order)
+};
+template <int OFF> __device__ __forceinline__ lane_pair lane_swap(float v) {
+  static_assert(OFF == 16 || OFF == 32, "row swaps");
+  const uint32_t u = __float_as_uint(v);
+  const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                           : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+// v + the value of the lane OFF apart (lane ^ OFF)
+template <int OFF> __device__ __forceinline__ float add_xor(float v) {
+  static_assert(OFF == 1 || OFF == 2 || OFF == 8 || OFF == 16 || OFF == 32, "see add_xor4 for 4");
+  if constexpr (OFF == 1) return v + lane_dpp<0xB1>(v);        // quad_perm [1,0,3,2]
+  else if constexpr (OFF == 2) return v + lane_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  else if constexpr (OFF == 8) return v + lane_dpp<0x128>(v);  // row_ror:8
+  else {
+    const lane_pair p = lane_swap<OFF>(v);
+    return p.a + p.b;
+  }
+}
+// the same 4 apart, for values equal within quads (1 and 2 apart already added): row_half_mirror
+__device__ __forceinline__ float add_xor4_quads(float v) { return v + lane_dpp<0x141>(v); }
+__device__ __forceinline__ float max_xor32(float v) {
+  const lane_pair p = lane_swap<32>(v);
+  return fmaxf(p.a, p.b);
+}
+
+// Sum over the 64 lanes of a wave, 32 apart first (every lane ends with the result). 4 apart: row_ror:4, since the values
+// have period 8 within a row by then.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v = add_xor<32>(v);
+  v = add_xor<16>(v);
+  v = add_xor<8>(v);
+  v += lane_dpp<0x124>(v);
+  v = add_xor<2>(v);
+  return add_xor<1>(v);
 }
 
 }  // namespace q35
