@@ -1296,29 +1296,36 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_prep_kernel(const float* __res
   if (tid == 0) recf[kFRecE / 4] = __expf(gam[kC - 1]);
 }
 
-// Operands of one chunk for one wave of the fp32 scan (CT column tiles of 16 per block).
+// Operands of one chunk for one state wave and one output wave of the fp32 scan (CT column tiles of 16 per block).
 template <int CT>
-struct F32Ops {
+struct F32State {
   f32x4 w[8];      // W rows 16 w + li, k chunks 0..7
-  f32x4 qe[8];     // Qe rows 16 w + li
-  f32x4 p[4];      // P row 16 w + li, position chunks 0..3 (chunks past w unused)
   f32x4 kt[2][4];  // Kt rows 32 w + 16 i + li, position chunks 0..3
   f32x4 u[CT];     // U rows 16 w + 4 lg + r, the block's columns
   float eg;
 };
+struct F32Out {
+  f32x4 qe[8];  // Qe rows 16 w + li
+  f32x4 p[4];   // P rows 16 w + li, position chunks 0..3 (chunks past w unused)
+};
 
 // CT column tiles of 16 per block: 8 / CT blocks per (row, head). The launcher takes CT = 2 when 8 blocks per (row,
-// head) would not all be resident at once (one block per CU: 316 VGPRs); the W, Qe, P, Kt operands are then loaded
-// once for two column tiles.
+// head) would not all be resident at once (one block per CU); the W, Qe, P, Kt operands are then loaded once for two
+// column tiles.
+// Eight waves, two per SIMD: waves 0-3 carry the state chain (V = U - W S, S <- e^g S + Kt V), waves 4-7 form the outputs
+// (Qe S between the step's two barriers, P V after the second). One wave per SIMD doing both ran its 224 fp32 MFMAs of a
+// chunk (3.0 us at full rate) one dependent phase after the other. Three rows x 2048 tokens, 16 heads, under the profiler:
+// 205 -> 188 us with eight waves (5.9 us a chunk), 162 with the records touched ahead; the chain without any load 130.
 template <int CT>
-__global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __restrict__ ws, const float* s_in,
+__global__ __launch_bounds__(512, 1) void gdn_f32_scan_kernel(const char* __restrict__ ws, const float* s_in,
                                                               float* s_out, float* __restrict__ o, int T, int NC,
                                                               int H, int B, int Hk, GdnFront fe) {
   constexpr int NSL = 8 / CT;      // blocks (slices) per (row, head)
-  __shared__ f32x4 sS[8][CT][64];  // state row tiles (D layout) of the four waves
+  __shared__ f32x4 sS[8][CT][64];  // state row tiles (D layout) of the four state waves
   __shared__ f32x4 sV[4][CT][64];  // V row tiles
   const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int w = wave & 3;
   const int li = lane & 15, lg = lane >> 4;
   // the blocks of one (row, head) read the same records: place them on one XCD (block i runs on XCD i % 8)
   const int nunits = H * B, L = blockIdx.x;
@@ -1336,6 +1343,76 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __rest
   for (int ct = 0; ct < CT; ++ct) col[ct] = 16 * (CT * sl + ct) + li;
   const char* rec0 = ws + (size_t)unit * NC * kFRecBytes;
   const size_t sbase = (size_t)unit * kD * kD;
+  auto rec = [&](int c) { return rec0 + (size_t)min(c, NC - 1) * kFRecBytes; };
+  auto frag = [&](const char* r, size_t part, int i) { return reinterpret_cast<const f32x4*>(r + part)[i * 64 + lane]; };
+
+  if (wave >= 4) {
+    auto load = [&](int c, F32Out& op) {
+      const char* r = rec(c);
+#pragma unroll
+      for (int kc = 0; kc < 8; ++kc) op.qe[kc] = frag(r, kFRecQ, 8 * w + kc);
+#pragma unroll
+      for (int kc = 0; kc < 4; ++kc) op.p[kc] = frag(r, kFRecP, 4 * w + kc);
+    };
+    auto step = [&](int c, const F32Out& op) {
+      lds_barrier();  // the chunk's incoming state is in sS
+      f32x4 oacc[CT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) oacc[ct] = zero4();
+#pragma unroll
+      for (int kc = 0; kc < 8; ++kc)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) oacc[ct] = mm_k16(op.qe[kc], sS[kc][ct][lane], oacc[ct]);
+      lds_barrier();  // V is in sV; the state waves may write the next state
+      f32x4 Vb[CT][4];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) Vb[ct][kc] = sV[kc][ct][lane];
+#pragma unroll
+      for (int kc = 0; kc < 4; ++kc)
+        if (kc <= w) {
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) oacc[ct] = mm_k16(op.p[kc], Vb[ct][kc], oacc[ct]);
+        }
+      const int tb = kC * c + 16 * w + 4 * lg;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (tb + r < T) o[(((size_t)b * T + tb + r) * H + h) * kD + col[ct]] = oacc[ct][r];
+    };
+    // The record of two chunks on into the L2: a step's loads are issued one step ahead, which hides an L2 round trip but
+    // not all of HBM's (3 rows x 2048 tokens: 178 us, 137 with every record already in the L2, 162 with this; touching
+    // three chunks on is no faster). The blocks of a unit share an XCD, so each touches its part of the lines, one dword
+    // per lane, consumed a step later.
+    constexpr int kLines = (int)(kFRecBytes / 128), kPart = (kLines + NSL - 1) / NSL;
+    static_assert(kPart <= 512, "two lines per thread of the output waves");
+    const bool shared_l2 = CT == 2 && (nunits & 7) == 0;  // (one column tile, at most two rows: no gain, 88 and 90 us)
+    const int l0 = sl * kPart + (int)threadIdx.x - 256, lend = min((sl + 1) * kPart, kLines);
+    float t0 = 0.f, t1 = 0.f;
+    auto touch = [&](int c) {
+      asm volatile("" ::"v"(t0), "v"(t1));  // (the previous touch has landed)
+      if (!shared_l2 || c >= NC) return;
+      const char* r = rec(c);
+      if (l0 < lend) t0 = *reinterpret_cast<const float*>(r + (size_t)l0 * 128);
+      if (l0 + 256 < lend) t1 = *reinterpret_cast<const float*>(r + (size_t)(l0 + 256) * 128);
+    };
+    F32Out o0, o1;
+    load(0, o0);
+    for (int c = 0; c < NC; c += 2) {
+      load(c + 1, o1);
+      touch(c + 2);
+      step(c, o0);
+      if (c + 1 < NC) {
+        load(c + 2, o0);
+        touch(c + 3);
+        step(c + 1, o1);
+      }
+    }
+    asm volatile("" ::"v"(t0), "v"(t1));
+    return;
+  }
 
   f32x4 S[CT][2];
 #pragma unroll
@@ -1346,46 +1423,33 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __rest
       for (int r = 0; r < 4; ++r)
         S[ct][i][r] = s_in ? s_in[sbase + (size_t)(32 * w + 16 * i + 4 * lg + r) * kD + col[ct]] : 0.f;
 
-  auto load = [&](int c, F32Ops<CT>& op) {
-    const char* rec = rec0 + (size_t)min(c, NC - 1) * kFRecBytes;
-    auto frag = [&](size_t part, int i) { return reinterpret_cast<const f32x4*>(rec + part)[i * 64 + lane]; };
+  auto load = [&](int c, F32State<CT>& op) {
+    const char* r = rec(c);
 #pragma unroll
-    for (int kc = 0; kc < 8; ++kc) {
-      op.w[kc] = frag(kFRecW, 8 * w + kc);
-      op.qe[kc] = frag(kFRecQ, 8 * w + kc);
-    }
+    for (int kc = 0; kc < 8; ++kc) op.w[kc] = frag(r, kFRecW, 8 * w + kc);
 #pragma unroll
-    for (int kc = 0; kc < 4; ++kc) op.p[kc] = frag(kFRecP, 4 * w + kc);
+    for (int ct = 0; ct < CT; ++ct) op.u[ct] = frag(r, kFRecU, 8 * w + CT * sl + ct);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int kc = 0; kc < 4; ++kc) op.kt[i][kc] = frag(kFRecK, 4 * (2 * w + i) + kc);
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) op.u[ct] = frag(kFRecU, 8 * w + CT * sl + ct);
-    op.eg = *reinterpret_cast<const float*>(rec + kFRecE);
+      for (int kc = 0; kc < 4; ++kc) op.kt[i][kc] = frag(r, kFRecK, 4 * (2 * w + i) + kc);
+    op.eg = *reinterpret_cast<const float*>(r + kFRecE);
   };
 
-  auto step = [&](int c, const F32Ops<CT>& op) {
+  auto step = [&](const F32State<CT>& op) {
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       sS[2 * w][ct][lane] = S[ct][0];
       sS[2 * w + 1][ct][lane] = S[ct][1];
     }
     lds_barrier();
-    f32x4 ws_[CT], oacc[CT];
+    f32x4 ws_[CT];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      ws_[ct] = zero4();
-      oacc[ct] = zero4();
-    }
+    for (int ct = 0; ct < CT; ++ct) ws_[ct] = zero4();
 #pragma unroll
-    for (int kc = 0; kc < 8; ++kc)
+    for (int kc = 0; kc < 8; ++kc)  // (the wave's own tiles from LDS too: a select per tile became a branch per read)
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        const f32x4 sb = (kc >> 1) == w ? S[ct][kc & 1] : sS[kc][ct][lane];
-        ws_[ct] = mm_k16(op.w[kc], sb, ws_[ct]);
-        oacc[ct] = mm_k16(op.qe[kc], sb, oacc[ct]);
-      }
+      for (int ct = 0; ct < CT; ++ct) ws_[ct] = mm_k16(op.w[kc], sS[kc][ct][lane], ws_[ct]);
     f32x4 vn[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
@@ -1398,32 +1462,24 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __rest
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-      for (int kc = 0; kc < 4; ++kc) Vb[ct][kc] = kc == w ? vn[ct] : sV[kc][ct][lane];
+      for (int kc = 0; kc < 4; ++kc) Vb[ct][kc] = sV[kc][ct][lane];
+    f32x4 sn[2][CT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sn[i][ct][r] = op.eg * S[ct][i][r];
 #pragma unroll
     for (int kc = 0; kc < 4; ++kc)
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-        if (kc <= w) oacc[ct] = mm_k16(op.p[kc], Vb[ct][kc], oacc[ct]);
-    const int tb = kC * c + 16 * w + 4 * lg;
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+        for (int ct = 0; ct < CT; ++ct) sn[i][ct] = mm_k16(op.kt[i][kc], Vb[ct][kc], sn[i][ct]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (tb + r < T) o[(((size_t)b * T + tb + r) * H + h) * kD + col[ct]] = oacc[ct][r];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      f32x4 sn[CT];
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sn[ct][r] = op.eg * S[ct][i][r];
-#pragma unroll
-      for (int kc = 0; kc < 4; ++kc)
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) sn[ct] = mm_k16(op.kt[i][kc], Vb[ct][kc], sn[ct]);
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) S[ct][i] = sn[ct];
-    }
+      for (int ct = 0; ct < CT; ++ct) S[ct][i] = sn[i][ct];
   };
 
   // front-end form: the carried conv state of this block's channels (16 CT of the head's v channels, and for the first
@@ -1445,7 +1501,7 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __rest
     }
   }
 
-  F32Ops<CT> o0, o1;
+  F32State<CT> o0, o1;
   load(0, o0);
   if (fstate) {
 #pragma unroll
@@ -1453,10 +1509,10 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __rest
   }
   for (int c = 0; c < NC; c += 2) {
     load(c + 1, o1);
-    step(c, o0);
+    step(o0);
     if (c + 1 < NC) {
       load(c + 2, o0);
-      step(c + 1, o1);
+      step(o1);
     }
   }
   if (s_out) {
@@ -1474,10 +1530,10 @@ __global__ __launch_bounds__(256, 1) void gdn_f32_scan_kernel(const char* __rest
 static void gdn_f32_scan_launch(const char* ws, const float* s_in, float* s_out, float* o, int T, int NC, int H,
                                 int B, int Hk, const GdnFront& fe, hipStream_t st) {
   if (8 * H * B <= 256)
-    hipLaunchKernelGGL(gdn_f32_scan_kernel<1>, dim3((unsigned)(8 * H * B)), dim3(256), 0, st, ws, s_in, s_out, o, T,
+    hipLaunchKernelGGL(gdn_f32_scan_kernel<1>, dim3((unsigned)(8 * H * B)), dim3(512), 0, st, ws, s_in, s_out, o, T,
                        NC, H, B, Hk, fe);
   else
-    hipLaunchKernelGGL(gdn_f32_scan_kernel<2>, dim3((unsigned)(4 * H * B)), dim3(256), 0, st, ws, s_in, s_out, o, T,
+    hipLaunchKernelGGL(gdn_f32_scan_kernel<2>, dim3((unsigned)(4 * H * B)), dim3(512), 0, st, ws, s_in, s_out, o, T,
                        NC, H, B, Hk, fe);
 }
 
