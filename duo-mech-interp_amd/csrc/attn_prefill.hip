@@ -473,7 +473,7 @@ static int pf_schedule(int nqb, int Ls, int ks_per, int64_t n_other, int gw, int
   // past 256 K blocks (a simulation of about 10 ms) the whole blocks spread evenly however long the longest is
   if ((int64_t)pf_items(nqb, Ls, false) * n_other > ((int64_t)1 << 18)) return 0;
   struct Key {
-    int nqb, gw, cus;
+    int nqb, gw, cus, ks_per;
     int64_t n_other;
   };
   static std::mutex mu;
@@ -483,7 +483,9 @@ static int pf_schedule(int nqb, int Ls, int ks_per, int64_t n_other, int gw, int
   {
     std::lock_guard<std::mutex> lock(mu);
     for (int i = 0; i < nkeys; ++i)
-      if (keys[i].nqb == nqb && keys[i].gw == gw && keys[i].cus == cus && keys[i].n_other == n_other) return vals[i];
+      if (keys[i].nqb == nqb && keys[i].gw == gw && keys[i].cus == cus && keys[i].ks_per == ks_per &&
+          keys[i].n_other == n_other)
+        return vals[i];
   }
   double best = pf_dispatch_time(nqb, 0, false, n_other, cus);
   int pick = 0;
@@ -505,7 +507,7 @@ static int pf_schedule(int nqb, int Ls, int ks_per, int64_t n_other, int gw, int
     if (ks_per + 2.0 + 0.01 * gw * (double)(parts * n_other) < best) pick = 2;
   }
   std::lock_guard<std::mutex> lock(mu);
-  keys[next] = Key{nqb, gw, cus, n_other};
+  keys[next] = Key{nqb, gw, cus, ks_per, n_other};
   vals[next] = pick;
   next = (next + 1) % 32;
   nkeys = nkeys < 32 ? nkeys + 1 : 32;
@@ -1092,7 +1094,7 @@ static int device_cus() {
 // queries ([B, T, Hq, D] bf16), then the partials of the split blocks ([pairs][2 halves][wave] x kPartFloats fp32) or of the
 // key runs ([query block and (row, kv head, group)][NS runs][wave]).
 struct PfLayout {
-  size_t q_off, part_off, total;
+  size_t q_off, part_off, base, total;  // base: without room for key runs
   int64_t npairs;
   int ks_per, ks_ns;  // key runs: the shortest run, the most runs of a query block (0: not an option)
 };
@@ -1111,6 +1113,7 @@ static PfLayout pf_layout(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, bool fp
   l.ks_per = pf_ks_len((int)nqb, B * Hkv * (G / GW), kKsSlots, &ns);
   l.ks_ns = l.ks_per ? ns : 0;
   const size_t runs = (size_t)l.ks_ns * nqb * B * Hkv * (G / GW), halves = (size_t)2 * l.npairs;
+  l.base = (l.part_off + halves * GW * kPartFloats * sizeof(float) + 255) / 256 * 256;
   l.total = (l.part_off + (runs > halves ? runs : halves) * GW * kPartFloats * sizeof(float) + 255) / 256 * 256;
   return l;
 }
@@ -1144,14 +1147,13 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
   const int Lmax = pf_split_len((int)nqb);
   const int64_t n_other = B * Hkv * ngroups;
   if ((int64_t)pf_items((int)nqb, Lmax, false) * n_other > 0x7fffffff) return Q35_EUNSUPPORTED;
-  if (pf_layout(B, T, Hq, Hkv, FP, Lmax).npairs > 0x7fffffff) return Q35_EUNSUPPORTED;
-  // the workspace as the size functions report it (the split case), checked before any HIP call
-  if (!workspace || workspace_bytes < pf_layout(B, T, Hq, Hkv, FP, Lmax).total || ((uintptr_t)workspace & 255))
-    return Q35_EWORKSPACE;
+  // the workspace, checked before any HIP call: the split case's, or as the size functions report it with room for runs
+  const PfLayout lay0 = pf_layout(B, T, Hq, Hkv, FP, Lmax);
+  if (lay0.npairs > 0x7fffffff) return Q35_EUNSUPPORTED;
+  if (!workspace || workspace_bytes < lay0.base || ((uintptr_t)workspace & 255)) return Q35_EWORKSPACE;
   // the first HIP call: the device's compute units decide the split and the work order
   const int cus = device_cus();
-  const PfLayout lay0 = pf_layout(B, T, Hq, Hkv, FP, Lmax);
-  const int sched = pf_schedule((int)nqb, Lmax, lay0.ks_per, n_other, GW, cus);
+  const int sched = pf_schedule((int)nqb, Lmax, workspace_bytes < lay0.total ? 0 : lay0.ks_per, n_other, GW, cus);
   const bool runs = sched == 2;
   const int Ls = sched == 1 ? Lmax : 0;
   const PfLayout lay = pf_layout(B, T, Hq, Hkv, FP, Ls);
@@ -1359,8 +1361,9 @@ extern "C" int q35_gated_attn_prefill_cached_proj(const float* y, int64_t ldy, c
   const int64_t nqb = (T + kBQ - 1) / kBQ, ntk = (T + kBN - 1) / kBN;
   const int64_t nblocks = nqb * B * Hkv * ngroups;
   if (nblocks > 0x7fffffff || ntk * (1 + G) + max_len / kBN > 0x7fffffff) return Q35_EUNSUPPORTED;
-  const size_t need = q35_gated_attn_prefill_cached_proj_workspace_bytes(B, T, Hq, Hkv, D, max_len);
-  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return Q35_EWORKSPACE;
+  if (q35_gated_attn_prefill_cached_proj_workspace_bytes(B, T, Hq, Hkv, D, max_len) == 0 || !workspace ||
+      workspace_bytes < pfc_proj_part_off(B, T, Hq, Hkv, max_len) || ((uintptr_t)workspace & 255))
+    return Q35_EWORKSPACE;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   __bf16* vt = static_cast<__bf16*>(workspace);
   __bf16* qr = reinterpret_cast<__bf16*>(static_cast<char*>(workspace) + pfc_proj_q_off(B, Hkv, max_len));
@@ -1379,7 +1382,8 @@ extern "C" int q35_gated_attn_prefill_cached_proj(const float* y, int64_t ldy, c
   }
 #undef Q35_KVC_LAUNCH
   // the queries arrive rotated (rot 0 in the main kernel); keys from the cache, the gate from y
-  const int runs = pfc_runs(B, T, Hq, Hkv, max_len);
+  const bool room = workspace_bytes >= q35_gated_attn_prefill_cached_proj_workspace_bytes(B, T, Hq, Hkv, D, max_len);
+  const int runs = room ? pfc_runs(B, T, Hq, Hkv, max_len) : 1;
   float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + pfc_proj_part_off(B, T, Hq, Hkv, max_len));
 #define Q35_PFCP_LAUNCH(GG)                                                                                        \
   hipLaunchKernelGGL((runs > 1 ? attn_prefill_kernel<GG, false, true, true>                                        \

@@ -65,6 +65,27 @@ def test_prefill_key_runs(B, T, Hq, Hkv):
     assert torch.equal(out, q35hip.gated_attention_prefill(*args))
 
 
+def test_prefill_workspace_without_room_for_runs():
+    """A workspace with room for K, V^T and the split halves only (T 512, 8 query / 2 kv heads: 16 pairs of halves of
+    four waves) is taken, by another schedule; one byte less is refused before any launch."""
+    dev = device()
+    T = 512
+    inp = workloads.to_device(workloads.attn_prefill_inputs(B=1, T=T, seed=3), dev)
+    cos, sin = (t.to(dev) for t in _tables(T))
+    full = q35hip.gated_attention_prefill(inp["q"], inp["k"], inp["v"], inp["gate"], cos, sin)
+    need = 2 * 2 * T * 256 * 2 + 2 * 16 * 4 * (8192 + 128) * 4
+    L = q35hip.lib()
+    assert L.q35_gated_attn_prefill_workspace_bytes(1, T, 8, 2, 256) > need
+    ws, out = torch.empty(need, dtype=torch.uint8, device=dev), torch.empty_like(full)
+    args = [inp[n].data_ptr() for n in ("q", "k", "v", "gate")] + [cos.data_ptr(), sin.data_ptr(), 0, out.data_ptr(),
+                                                                  1, T, 8, 2, 256, 64, 256 ** -0.5, ws.data_ptr()]
+    announce("attn prefill small workspace")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert L.q35_gated_attn_prefill(*args, need - 1, stream) == 3
+    assert L.q35_gated_attn_prefill(*args, need, stream) == 0
+    assert oracle.rel_err(out.float().cpu(), full.float().cpu()) <= 4e-3  # bf16 outputs of the same fp32 sums
+
+
 def test_prefill_full_size():
     """B = 1, T = 4096, causal, 8 q / 2 kv heads, head dim 256, RoPE theta 1e7 on dims 0..63, sigmoid gate."""
     dev = device()
