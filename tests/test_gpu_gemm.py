@@ -252,3 +252,23 @@ def test_gemm_q8_few_rows(x_form, M, N, K, gs):
     if N % 16 == 0:
         b = ops.gemm_q8(xin, qd, sd, epilogue="swiglu", pushes=ops.pack_pushes(pushes, dev), T=T, split_out=True)
         assert torch.equal(b, ops.split_activations(a))
+
+
+# the register-staged kernel's tile order: 297 tiles of 64 rows (8 x 37 + 1), and 8300 rows, where fp32 and split x take
+# 1170 tiles of 64 rows and bf16 x 585 of 128, each with ragged last tiles in both directions
+@pytest.mark.parametrize("x_form", ["fp32", "split", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(2085, 1050, 128), (8300, 1030, 128)])
+def test_gemm_q8_tile_order(x_form, M, N, K):
+    """Every output against the fp64 product of the dequantised weights: x = hi + lo drops at most 2^-17 of each value
+    and a fp32 sum of K products (the kernel's two, hi and lo) 2 K roundings of 2^-24, both of sum |x w|."""
+    dev = device()
+    q, s = _q8g(N, K, M + N + K)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(K + M)) * 3.0
+    if x_form == "bf16":
+        x = x.to(torch.bfloat16)
+    xd = x.to(dev)
+    w = omlp.q8_dequant(q, s).double()
+    announce(f"gemm_q8 tile order {x_form} M{M} N{N} K{K}")
+    y = ops.gemm_q8(ops.split_activations(xd) if x_form == "split" else xd, q.to(dev), s.to(dev)).cpu()
+    bound = (2.0 ** -17 + 2 * K * 2.0 ** -24) * (x.double().abs() @ w.abs().T)
+    assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
