@@ -947,8 +947,12 @@ static int gemm_rs_launch(const float* x, int64_t ldx, const int8_t* W, const fl
                           int64_t M, int64_t N, int64_t K, int epilogue, bool gs, const q35_push* pushes, int64_t npush,
                           int64_t T, int64_t moff, int ys, const GemmCap& cap, hipStream_t st) {
   const int64_t nbn = (N + kGN - 1) / kGN;
-  // 128-row tiles when they still give at least two blocks per compute unit, else 64-row tiles
-  const bool big = ((M + 127) / 128) * nbn >= 512;
+  // bf16 x: 128-row tiles when they still give at least two blocks per compute unit (8192 / 16384 x 1024 x 2048: 58 /
+  // 115 us, with 64 rows 70 / 128). The other forms hold twice the MFMAs and more registers per tile (198 VGPRs, two
+  // blocks per CU where 64 rows let three in), and 64-row tiles are the faster ones or equal at every size measured
+  // (1024 x 3584 accumulating, split x, 8192 / 9000 / 12288 / 32768 rows: 193 / 196 / 252 / 633 us, with 128 rows
+  // 204 / 254 / 273 / 692; at worst 3 % behind where 128-row tiles fill exactly one round, fp32 x at 8192 rows).
+  const bool big = XF == 2 && ((M + 127) / 128) * nbn >= 512;
   const int BM = big ? 128 : 64;
   const int64_t nblocks = ((M + BM - 1) / BM) * nbn;
   if (nblocks > 0x7fffffff) return Q35_EUNSUPPORTED;
@@ -960,7 +964,9 @@ static int gemm_rs_launch(const float* x, int64_t ldx, const int8_t* W, const fl
   else if (epilogue == kGemmAccumulate) Q35_GEMM_LAUNCH(BMV, kGemmAccumulate, G); \
   else Q35_GEMM_LAUNCH(BMV, kGemmSwiglu, G);
   if (big) {
-    if (gs) { Q35_GEMM_EPI(128, true) } else { Q35_GEMM_EPI(128, false) }
+    if constexpr (XF == 2) {
+      if (gs) { Q35_GEMM_EPI(128, true) } else { Q35_GEMM_EPI(128, false) }
+    }
   } else {
     if (gs) { Q35_GEMM_EPI(64, true) } else { Q35_GEMM_EPI(64, false) }
   }
