@@ -1075,9 +1075,9 @@ def gemm_q8(x, W, w_scale, out=None, epilogue="store", pushes=None, T=1, split_o
     accumulates into out, "swiglu" treats W's rows as interleaved (gate, up) pairs and writes
     silu(gate) * up with the neuron pushes (pack_pushes) applied, out [M, N / 2]. x may also be the int32 words of
     activations already split (add_rmsnorm_(..., split=True), split_activations): the same product, bitwise, without
-    the split in the kernel; or bf16 (the lo products skipped: the product of x.float() bitwise where that runs the register-staged
-    kernel, N < 2048 or K > 2048, and to fp32 rounding on the wide shapes). split_out=True (SwiGLU only) writes out as the int32 words of the split layout, the
-    input of the next gemm_q8. capture: as for gemv (the fp32 activations, whatever the layout of out). Returns out."""
+    the split in the kernel; or bf16 (the lo products skipped: the product of x.float() bitwise for N < 2048 or K > 2048,
+    where both take the same kernel, and to fp32 rounding on the wide shapes). split_out=True (SwiGLU only) writes out
+    as the int32 words of the split layout, the input of the next gemm_q8. capture: as for gemv (the fp32 activations, whatever the layout of out). Returns out."""
     e = _EPI[epilogue]
     if split_out:
         if e != 2:

@@ -493,10 +493,10 @@ int q35_gemm_q8_split(const void* xs, int64_t ldx, const int8_t* W, int w_dtype,
 
 /*
  * q35_gemm_q8 on bf16 x (the attention output, read without a conversion to fp32): xb [M, ldx] bf16, 16-byte
- * aligned, ldx a multiple of 8. Runs on the register-staged kernel with only the hi products issued (the hi parts are
- * x, the lo parts zero): bitwise q35_gemm_q8 on the fp32 values of x where that also runs the register-staged kernel
- * (N < 2048 or K > 2048), equal to fp32 rounding elsewhere (the DMA kernel sums K in another grouping). Same
- * reference lines.
+ * aligned, ldx a multiple of 8. Runs on the few-row and register-staged kernels with only the hi products issued (the hi
+ * parts are x, the lo parts zero): bitwise q35_gemm_q8 on the fp32 values of x for N < 2048 or K > 2048, where both
+ * take the same kernel, equal to fp32 rounding elsewhere (the DMA kernel sums K in another grouping). Same reference
+ * lines.
  */
 int q35_gemm_q8_bf16(const void* xb, int64_t ldx, const int8_t* W, int w_dtype, const float* w_scale, float* y,
                      int64_t ldy, int64_t M, int64_t N, int64_t K, int epilogue, const q35_push* pushes,
