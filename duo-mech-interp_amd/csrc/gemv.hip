@@ -17,8 +17,8 @@
 // the waves in LDS. Epilogues: store, accumulate into y (the residual add after down_proj), or SwiGLU over interleaved
 // (gate, up) row pairs with the neuron pushes applied (gate_up_proj). With group scales a lane's 16 weights of a K step
 // lie in one group (group 2 step + slot / 8), so the lane scales its partial sum of the step once.
-// TL (fp32 weights with more tiles than kGemvMaxBlocks): a block takes tiles blockIdx.x, blockIdx.x + gridDim.x, ...;
-// the next tile's weights are issued before the current tile's products when a wave has one K step per tile (two
+// TL (more tiles than kGemvMaxBlocks, fp32 weights or the gated-norm prologue): a block takes tiles blockIdx.x,
+// blockIdx.x + gridDim.x, ...; the next tile's weights are issued before the current tile's products when a wave has one K step per tile (two
 // register sets), else before its reduction.
 // What a block waits for, beside the weights: the x operands go out ahead of the weights and are consumed in straight-line
 // code (consumed in a loop, their wait became a wait for the weights too: gate/up at 3 rows 6.9 -> 6.4 us), rows of x are
@@ -512,12 +512,12 @@ namespace {
 // Blocks of 16 output rows at which a product is split over K: below this many, an accumulating product without the
 // norm splits its K steps so that blocks x splits reaches it (one block per CU of the MI355X).
 constexpr int64_t kGemvSplitTarget = 256;
-// Grid cap: an fp32 product with more 16-row tiles loops each block over tiles blockIdx.x, + gridDim.x, ... (x staged
-// once per block; four 4-wave blocks per CU at 128 VGPRs), an int8 one (the LM head: 9496) runs the tile loop of
-// gemv_mfma.hip. The products with fewer tiles take one tile per block (measured faster for them).
-constexpr int64_t kGemvMaxBlocks = 1024;
 // Rows of x from which an int8 product runs on the matrix core: the times on both sides of the line are in gemv_mfma.hip.
 constexpr int64_t kGemvMfmaRows = 4;
+// Whether a product with more tiles than kGemvMaxBlocks loops its blocks over them in the form of this file (TL): fp32
+// weights, and int8 ones behind the gated norm, which the tile loop of gemv_mfma.hip does not have. The grid is capped
+// for exactly these.
+constexpr bool gemv_loops(bool fp32, bool gn) { return fp32 || gn; }
 
 template <typename TW, int EPI, int U, bool NORM, bool GS, bool GN, int R = 4>
 void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale, float* y, int64_t ldy, int64_t M,
@@ -532,27 +532,30 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
   constexpr int R8 = R > 2 ? 2 : R;
   const int re = mp == 8 ? R8 : R;
   const int64_t ntiles = (N + 4 * re - 1) / (4 * re);
-  const dim3 grid((unsigned)(ntiles < kGemvMaxBlocks ? ntiles : kGemvMaxBlocks), (unsigned)nsplit), block(64 * nw);
+  // kFew: int8 products of kGemvMfmaRows rows or more run gemv_mfma.hip; the 4-row tiles (R 1) stay here for every M.
+  // The tile loop is compiled for every form that can have more tiles than blocks (the conv epilogue's entry point and
+  // the 4-row tiles' launcher bound N), and the grid is capped only with it.
+  constexpr bool kFew = sizeof(TW) == 1 && R > 1;
+  constexpr bool kLoop = EPI != kEpiConv && R > 1 && gemv_loops(sizeof(TW) == 4, GN);
+  const bool loop = kLoop && ntiles > kGemvMaxBlocks;
+  const dim3 grid((unsigned)(loop ? kGemvMaxBlocks : ntiles), (unsigned)nsplit), block(64 * nw);
 #define Q35_GEMV(MP, TL)                                                                                           \
   hipLaunchKernelGGL((gemv_kernel<TW, MP, EPI, U, NORM, GS, TL, (MP == 8 ? R8 : R), GN>), grid, block, lds, st, x, \
                      ldx, W, wscale, y, ldy, (int)M, (int)N, (int)K, pushes, npush, (int)T, na.xadd, na.nw, na.eps,   \
                      na.xout, na.aux)
-  // int8 products of kGemvMfmaRows rows or more, and those with more tiles than blocks, run gemv_mfma.hip; the 4-row
-  // tiles (R 1) stay here for every M
-  constexpr bool kFew = sizeof(TW) == 1 && R > 1;
-  if constexpr (EPI != kEpiConv && !kFew && R > 1) {
-    if (ntiles > kGemvMaxBlocks) {
+  if constexpr (kLoop) {
+    if (loop) {
       switch (mp) {
         case 1: Q35_GEMV(1, true); break;
         case 2: Q35_GEMV(2, true); break;
         case 3: Q35_GEMV(3, true); break;
-        case 4: Q35_GEMV(4, true); break;
-        default: if constexpr (U <= 2) Q35_GEMV(8, true); break;  // 8 rows: U <= 2 (gemv_launch)
+        case 4: if constexpr (!kFew) Q35_GEMV(4, true); break;
+        default: if constexpr (!kFew && U <= 2) Q35_GEMV(8, true); break;  // 8 rows: U <= 2 (gemv_launch)
       }
       return;
     }
   }
-  // one tile per block (the conv epilogue's entry point bounds N)
+  // one tile per block
   switch (mp) {
     case 1: Q35_GEMV(1, false); break;
     case 2: Q35_GEMV(2, false); break;
@@ -598,7 +601,7 @@ int gemv_launch(const float* x, int64_t ldx, const TW* W, const float* wscale, f
   const int nw = bsteps <= 4 ? 4 : 8;
   const int64_t per_wave = (bsteps + nw - 1) / nw;
   if constexpr (sizeof(TW) == 1) {
-    if (M >= kGemvMfmaRows || (EPI != kEpiConv && !GN && nsplit == 1 && nblk > kGemvMaxBlocks))
+    if (M >= kGemvMfmaRows || (EPI != kEpiConv && !gemv_loops(false, GN) && nsplit == 1 && nblk > kGemvMaxBlocks))
       return gemv_mfma_run(NORM, GN, GS, EPI, x, ldx, W, wscale, y, ldy, M, N, K, pushes, npush, T, (int)nsplit, na, st);
   }
   // more than 4 rows of x: at most two K steps per wave in flight (four spill the registers of 8 rows)

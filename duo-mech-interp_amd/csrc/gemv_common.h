@@ -9,6 +9,10 @@ enum GemvEpi : int { kEpiStore = 0, kEpiAccumulate = 1, kEpiSwiglu = 2, kEpiConv
 constexpr int kEpiAccumulateFixed = 4;  // entry-point code: accumulate, every output summed in one fixed order
 constexpr int kGemvConvMaxK = 8;  // conv taps supported by the conv epilogue
 constexpr int kGemvHead = 128;    // head size of the gated-norm prologue
+// Tiles of 16 output rows (8 for fp32 weights at more than 4 rows of x) past which blocks or waves loop over tiles, x staged
+// once per block (the LM head: 9496); products with fewer take one tile per block (measured faster for them). Also the
+// blocks of gemv.hip's loop: four of 4 waves per CU at 128 VGPRs.
+constexpr int64_t kGemvMaxBlocks = 1024;
 
 // Operands of the gated-norm prologue (GN) and of the conv epilogue (kEpiConv); unused by the other forms.
 struct GemvAux {

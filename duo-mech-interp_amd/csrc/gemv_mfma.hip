@@ -583,9 +583,7 @@ __global__ __launch_bounds__(256, 2) void gemv_tiles_kernel(const float* __restr
   }
 }
 
-// Tiles of 16 rows past which each wave loops over whole tiles (gemv_tiles_kernel; the LM head: 9496).
-constexpr int64_t kGemvTilesFrom = 1024;
-constexpr int64_t kGemvTileBlocks = 512;  // its blocks: two per CU
+constexpr int64_t kGemvTileBlocks = 512;  // blocks of gemv_tiles_kernel: two per CU
 
 // the matrix-core form (int8 weights, one 16-row tile per block)
 template <int EPI, int U, bool NORM, bool GS, bool GN>
@@ -638,7 +636,7 @@ static int gemv_mfma_epi(const float* x, int64_t ldx, const int8_t* W, const flo
                          int64_t M, int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T, int nsplit,
                          const GemvArgs& na, hipStream_t st) {
   if constexpr (EPI != kEpiConv && !GN) {
-    if (nsplit == 1 && (N + 15) / 16 > kGemvTilesFrom) {
+    if (nsplit == 1 && (N + 15) / 16 > kGemvMaxBlocks) {
       gemv_tiles_launch<EPI, NORM, GS>(x, ldx, W, wscale, y, ldy, M, N, K, pushes, npush, T, na, st);
       return hipGetLastError() == hipSuccess ? Q35_OK : Q35_ELAUNCH;
     }

@@ -374,3 +374,31 @@ def test_gemv_infinities_and_nan_stay_in_their_row(M, N):
         ok = ref[m].abs() < 3e38
         assert bool(y[m][ok].isfinite().all())
         assert oracle.rel_err(y[m][ok], ref[m][ok]) <= 2e-6
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
+@pytest.mark.parametrize("N,K", [(16384, 256), (16400, 2048), (33000, 1024)])
+@pytest.mark.parametrize("gs", [True, False])
+def test_gemv_gated_norm_many_tiles(M, N, K, gs):
+    """The gated-norm product up to, just past and well past as many 16-row tiles as the launch takes blocks, at every
+    epilogue: every output within K 2^-24 of its row's sum |h w| (fp32 sums; the prologue's rsqrt and silu are a few
+    roundings, taken as 16 more), from outputs that start as NaN (store) or known (add)."""
+    dev = device()
+    g = torch.Generator().manual_seed(N + K + M)
+    W, s = _weights_g128(N, K, N) if gs else _weights(N, K, torch.int8, N)
+    o, z = torch.randn(M, K, generator=g), torch.randn(M, K, generator=g)
+    nw, hs = 1.0 + 0.1 * torch.randn(128, generator=g), torch.rand(K // 128, generator=g) + 0.5
+    od = o.double().view(M, K // 128, 128)
+    h = (nw.double() * od * torch.rsqrt(od.pow(2).mean(-1, keepdim=True) + 1e-6)).view(M, K)
+    h = h * torch.nn.functional.silu(z.double()) * hs.double().repeat_interleave(128)
+    wd = omlp.q8_dequant(W, s).double()
+    ref, bound = h @ wd.T, (K + 16) * 2.0 ** -24 * (h.abs() @ wd.abs().T)
+    args = [t.to(dev) for t in (o, z, nw, W, s)]
+    base = torch.randn(M, N, generator=g)
+    for epi in ("store", "add", "add_fixed"):
+        announce(f"gemv_gated_norm M{M} N{N} K{K} gs {gs} {epi}")
+        out = torch.full((M, N), float("nan"), device=dev) if epi == "store" else base.to(dev)
+        ops.gemv_gated_norm(*args, out, head_scale=hs.to(dev), epilogue=epi)
+        exp = ref if epi == "store" else base.double() + ref
+        err = (out.cpu().double() - exp).abs()
+        assert bool((err <= bound + 2.0 ** -24 * exp.abs()).all()), f"{epi}: {int((~(err <= bound)).sum())} outputs off"
