@@ -17,8 +17,7 @@
 // the waves in LDS. Epilogues: store, accumulate into y (the residual add after down_proj), or SwiGLU over interleaved
 // (gate, up) row pairs with the neuron pushes applied (gate_up_proj). With group scales a lane's 16 weights of a K step
 // lie in one group (group 2 step + slot / 8), so the lane scales its partial sum of the step once.
-// TL (more tiles than kGemvMaxBlocks, fp32 weights or the gated-norm prologue): a block takes tiles blockIdx.x,
-// blockIdx.x + gridDim.x, ...; the next tile's weights are issued before the current tile's products when a wave has one K step per tile (two
+// TL (more tiles than kGemvMaxBlocks): a block takes tiles blockIdx.x, blockIdx.x + gridDim.x, ...; the next tile's weights are issued before the current tile's products when a wave has one K step per tile (two
 // register sets), else before its reduction.
 // What a block waits for, beside the weights: the x operands go out ahead of the weights and are consumed in straight-line
 // code (consumed in a loop, their wait became a wait for the weights too: gate/up at 3 rows 6.9 -> 6.4 us), rows of x are
@@ -463,14 +462,18 @@ __global__ __launch_bounds__(512) void gemv_kernel(const float* __restrict__ x, 
   }
   if constexpr (EPI == kEpiStore) {
     if (aux.amax) {  // uniform: every thread reaches the barrier
-      // the block's best key per row of x, then one device-scope atomic max per row
+      // the block's best key per row of x, then one device-scope atomic max per row. 1024 blocks' atomics on one slot take
+      // 10 us, so blocks of short tiles (U 1), which end together, first look whether the slot holds a larger key already
+      // (151,936 x 1024 at one row 39.8 -> 34.5 us); with long tiles the look costs more than it saves (32,768 x 3072 27.4 ->
+      // 30.2)
       __shared__ unsigned long long kbest[4 * R * MP];
       if (tid < 4 * R * MP) kbest[tid] = best_key;
       __syncthreads();
       if (tid < MP && tid < M) {
         unsigned long long k = 0ull;
         for (int rr = 0; rr < 4 * R; ++rr) k = kbest[rr * MP + tid] > k ? kbest[rr * MP + tid] : k;
-        if (k) __hip_atomic_fetch_max(aux.amax + tid, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (U > 1 ? k != 0ull : k > __hip_atomic_load(aux.amax + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+          __hip_atomic_fetch_max(aux.amax + tid, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
@@ -514,10 +517,30 @@ namespace {
 constexpr int64_t kGemvSplitTarget = 256;
 // Rows of x from which an int8 product runs on the matrix core: the times on both sides of the line are in gemv_mfma.hip.
 constexpr int64_t kGemvMfmaRows = 4;
-// Whether a product with more tiles than kGemvMaxBlocks loops its blocks over them in the form of this file (TL): fp32
-// weights, and int8 ones behind the gated norm, which the tile loop of gemv_mfma.hip does not have. The grid is capped
-// for exactly these.
-constexpr bool gemv_loops(bool fp32, bool gn) { return fp32 || gn; }
+// Whether an int8 product of 1 to 3 rows of x with more tiles than kGemvMaxBlocks runs the tile loop of gemv_mfma.hip (its
+// waves take whole tiles) rather than the one of this file (blocks take tiles). That one's time hardly grows with the
+// rows of x, but its 2048 waves (two blocks of four per CU) take ceil(tiles / 2048) tiles each, so a last round with few
+// tiles costs a full one, and it is slow over long rows of W; this one's blocks share a tile's K steps, and each ends on
+// an argmax atomic per row. A product and its argmax form run the same kernel, so that they give the same bits. Measured
+// on MI355X, group scales, us, here / there, plain or behind the norm (in parentheses with norm and argmax):
+//   1 row: 151,936 x 1024 31.5 / 35.2 (34.5 / 38.8), 65,536 x 1024 16.4 / 18.1 (22.0 / 21.6), 16,400 x 1024 6.2 / 8.4 (16.1 /
+//     12.2), 32,768 x 2048 15.6 / 17.8 (23.8 / 22.0), 20,480 x 4096 20.5 / 27.6 (26.2 / 31.5); with one K step per tile
+//     three of a block's four waves here have none: 151,936 x 256 18.4 / 17.7 (29.1 / 24.4), but 16,400 x 256 4.2 / 4.9;
+//   2 rows: 151,936 x 1024 (93 % of the last round's waves busy) 34.4 / 34.9 (38.8 / 38.4), 65,536 (100 %) 18.1 / 17.5
+//     (23.4 / 21.6), 40,008 (61 %) 12.2 / 14.3 (17.3 / 16.2), 16,400 (50 %) 7.1 / 8.5 (17.2 / 11.6), 50,000 x 3072 (76 %) 36.0 /
+//     41.0 (39.7 / 42.6);
+//   3 rows: 151,936 x 1024 40.5 / 35.3 (44.4 / 39.0), 65,536 20.7 / 17.4, 20,480 (62 %) 9.3 / 10.5 (14.6 / 13.3); 20,480 x
+//     4096 25.4 / 44.3, where the pieces of x leave one block per CU there.
+static bool gemv_tiles_on_mfma(int64_t M, int64_t K, int64_t ntiles, bool norm) {
+  using namespace q35;
+  const bool two = 2 * gemv_mfma_lds(4, M, K) <= kGemvLds;
+  const int64_t waves = 4 * kGemvTileBlocks, room = (ntiles + waves - 1) / waves * waves;
+  switch (M) {
+    case 1: return K < 512 && 10 * ntiles >= 9 * room;
+    case 2: return two && (norm || (K <= 2048 && 10 * ntiles >= 9 * room));
+    default: return two && (norm || K < 1024 || 10 * ntiles >= 7 * room);
+  }
+}
 
 template <typename TW, int EPI, int U, bool NORM, bool GS, bool GN, int R = 4>
 void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale, float* y, int64_t ldy, int64_t M,
@@ -536,7 +559,7 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
   // The tile loop is compiled for every form that can have more tiles than blocks (the conv epilogue's entry point and
   // the 4-row tiles' launcher bound N), and the grid is capped only with it.
   constexpr bool kFew = sizeof(TW) == 1 && R > 1;
-  constexpr bool kLoop = EPI != kEpiConv && R > 1 && gemv_loops(sizeof(TW) == 4, GN);
+  constexpr bool kLoop = EPI != kEpiConv && R > 1;
   const bool loop = kLoop && ntiles > kGemvMaxBlocks;
   const dim3 grid((unsigned)(loop ? kGemvMaxBlocks : ntiles), (unsigned)nsplit), block(64 * nw);
 #define Q35_GEMV(MP, TL)                                                                                           \
@@ -601,7 +624,8 @@ int gemv_launch(const float* x, int64_t ldx, const TW* W, const float* wscale, f
   const int nw = bsteps <= 4 ? 4 : 8;
   const int64_t per_wave = (bsteps + nw - 1) / nw;
   if constexpr (sizeof(TW) == 1) {
-    if (M >= kGemvMfmaRows || (EPI != kEpiConv && !gemv_loops(false, GN) && nsplit == 1 && nblk > kGemvMaxBlocks))
+    if (M >= kGemvMfmaRows || (EPI != kEpiConv && !GN && nsplit == 1 && nblk > kGemvMaxBlocks &&
+                               gemv_tiles_on_mfma(M, K, nblk, NORM)))
       return gemv_mfma_run(NORM, GN, GS, EPI, x, ldx, W, wscale, y, ldy, M, N, K, pushes, npush, T, (int)nsplit, na, st);
   }
   // more than 4 rows of x: at most two K steps per wave in flight (four spill the registers of 8 rows)

@@ -13,6 +13,17 @@ constexpr int kGemvHead = 128;    // head size of the gated-norm prologue
 // once per block (the LM head: 9496); products with fewer take one tile per block (measured faster for them). Also the
 // blocks of gemv.hip's loop: four of 4 waves per CU at 128 VGPRs.
 constexpr int64_t kGemvMaxBlocks = 1024;
+constexpr int64_t kGemvLds = 160 * 1024;  // LDS of a CU
+
+// The matrix-core form: blocks of its tile loop (two per CU), bytes of a wave's weight tile (16 rows x one K step), the
+// rows of x that it is compiled for, and the LDS of a block of nw waves that stages K columns of M rows (three bf16
+// pieces each).
+constexpr int64_t kGemvTileBlocks = 512;
+constexpr int kWTile = 16 * 256;
+constexpr int gemv_mfma_rows(int64_t M) { return M <= 5 ? (int)M : 8; }
+constexpr size_t gemv_mfma_lds(int nw, int64_t M, int64_t K) {
+  return (size_t)nw * kWTile + (size_t)3 * gemv_mfma_rows(M) * (2 * K + 16);
+}
 
 // Operands of the gated-norm prologue (GN) and of the conv epilogue (kEpiConv); unused by the other forms.
 struct GemvAux {

@@ -20,7 +20,6 @@
 namespace q35 {
 
 constexpr int gemv_ct(int mp) { return (3 * mp + 15) / 16; }  // MFMA column tiles of 3 pieces x mp rows
-constexpr int kWTile = 16 * 256;                              // bytes of a wave's weight tile (16 rows x one K step)
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
 // four consecutive values' pieces, packed in pairs: [piece][pair]
@@ -411,8 +410,9 @@ __global__ __launch_bounds__(512) void gemv_mfma_kernel(const float* __restrict_
 // crossed one per 16 rows. Rounds of four K steps (16 KB of weights per wave), each step's buffer refilled for the next
 // round, of this tile or the next, as soon as its products are done. Two blocks of four waves per CU: 128 KB in flight.
 // The pieces of a row are summed between the accumulator's columns with two lane exchanges. 151,936 x 1024 with group
-// scales and the argmax, at 1 / 3 / 5 / 8 rows: 39.4 / 40.6 / 41.2 / 44.8 us (160 MB: 3.6-4.1 TB/s), the block tile loop of
-// the fp32 form 40.5 / 47.7 / 105 / 107 us.
+// scales, the norm and the argmax, at 1 / 3 / 5 / 8 rows: 38.8 / 39.0 / 39.7 / 42.9 us (160 MB: 3.7-4.1 TB/s), the block tile
+// loop of gemv.hip 34.5 / 44.4 / 79.4 / 80.5; without the argmax 35.2 / 35.3 / 35.7 / 39.6 and 31.5 / 40.5 / 77.8 / 78.0.
+// Which of the two runs at 1 to 3 rows: gemv_tiles_on_mfma.
 template <int MP, int EPI, bool NORM, bool GS>
 __global__ __launch_bounds__(256, 2) void gemv_tiles_kernel(const float* __restrict__ x, int64_t ldx,
                                                             const int8_t* __restrict__ W,
@@ -583,21 +583,18 @@ __global__ __launch_bounds__(256, 2) void gemv_tiles_kernel(const float* __restr
   }
 }
 
-constexpr int64_t kGemvTileBlocks = 512;  // blocks of gemv_tiles_kernel: two per CU
-
 // the matrix-core form (int8 weights, one 16-row tile per block)
 template <int EPI, int U, bool NORM, bool GS, bool GN>
 void gemv_mfma_launch_u(const float* x, int64_t ldx, const int8_t* W, const float* wscale, float* y, int64_t ldy,
                         int64_t M, int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T, int nw,
                         int nsplit, const GemvArgs& na, hipStream_t st) {
-  const int mp = M <= 5 ? (int)M : 8;
   const int64_t spb = (K / 256 + nsplit - 1) / nsplit;
-  const size_t lds = (size_t)nw * kWTile + (size_t)3 * mp * (spb * 512 + 16);
+  const size_t lds = gemv_mfma_lds(nw, M, spb * 256);
   const dim3 grid((unsigned)((N + 15) / 16), (unsigned)nsplit), block(64 * nw);
 #define Q35_GEMV_MFMA(MP)                                                                                          \
   hipLaunchKernelGGL((gemv_mfma_kernel<MP, EPI, U, NORM, GS, GN>), grid, block, lds, st, x, ldx, W, wscale, y, ldy, \
                      (int)M, (int)N, (int)K, pushes, npush, (int)T, na.xadd, na.nw, na.eps, na.xout, na.aux)
-  switch (mp) {
+  switch (gemv_mfma_rows(M)) {
     case 1: Q35_GEMV_MFMA(1); break;
     case 2: Q35_GEMV_MFMA(2); break;
     case 3: Q35_GEMV_MFMA(3); break;
@@ -613,14 +610,13 @@ template <int EPI, bool NORM, bool GS>
 void gemv_tiles_launch(const float* x, int64_t ldx, const int8_t* W, const float* wscale, float* y, int64_t ldy,
                        int64_t M, int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T,
                        const GemvArgs& na, hipStream_t st) {
-  const int mp = M <= 5 ? (int)M : 8;
-  const size_t lds = (size_t)4 * kWTile + (size_t)3 * mp * (2 * K + 16);
+  const size_t lds = gemv_mfma_lds(4, M, K);
   const int64_t blocks = ((N + 15) / 16 + 3) / 4;
   const dim3 grid((unsigned)(blocks < kGemvTileBlocks ? blocks : kGemvTileBlocks)), block(256);
 #define Q35_GEMV_TILES(MP)                                                                                         \
   hipLaunchKernelGGL((gemv_tiles_kernel<MP, EPI, NORM, GS>), grid, block, lds, st, x, ldx, W, wscale, y, ldy, (int)M, \
                      (int)N, (int)K, pushes, npush, (int)T, na.xadd, na.nw, na.eps, na.xout, na.aux)
-  switch (mp) {
+  switch (gemv_mfma_rows(M)) {
     case 1: Q35_GEMV_TILES(1); break;
     case 2: Q35_GEMV_TILES(2); break;
     case 3: Q35_GEMV_TILES(3); break;

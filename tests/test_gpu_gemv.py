@@ -402,3 +402,40 @@ def test_gemv_gated_norm_many_tiles(M, N, K, gs):
         exp = ref if epi == "store" else base.double() + ref
         err = (out.cpu().double() - exp).abs()
         assert bool((err <= bound + 2.0 ** -24 * exp.abs()).all()), f"{epi}: {int((~(err <= bound)).sum())} outputs off"
+
+
+# int8 products past 1024 tiles at 1 to 3 rows, on both sides of the line between the two tile loops: half of a round of
+# waves (16,400 rows of W), all of one (32,762, ragged), short and long rows of W, and 4096 inputs, where three rows leave one
+# block per CU
+@pytest.mark.parametrize("M", [1, 2, 3])
+@pytest.mark.parametrize("N,K", [(16400, 256), (16400, 1024), (32762, 256), (32762, 1024), (16390, 4096)])
+@pytest.mark.parametrize("gs", [True, False])
+def test_gemv_tile_loops(M, N, K, gs):
+    """Store, accumulate, SwiGLU behind the norm and the argmax form against fp64: every output within K 2^-24 of its
+    row's sum |x w| (fp32 sums; 16 roundings more for the norm and the silu, whose slope is under 1.1)."""
+    dev = device()
+    g = torch.Generator().manual_seed(N + K + M)
+    W, s = _weights_g128(N, K, N) if gs else _weights(N, K, torch.int8, N)
+    x, nw, base = torch.randn(M, K, generator=g), 0.1 * torch.randn(K, generator=g), torch.randn(M, N, generator=g)
+    h = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6) * (1.0 + nw.double())
+    wd = omlp.q8_dequant(W, s).double()
+    eps = (K + 16) * 2.0 ** -24
+    ref, tol = x.double() @ wd.T, eps * (x.double().abs() @ wd.abs().T)
+    refn, toln = h @ wd.T, eps * (h.abs() @ wd.abs().T)
+    Wd, sd, xd, nwd = W.to(dev), s.to(dev), x.to(dev), nw.to(dev)
+    announce(f"gemv tile loops M{M} N{N} K{K} gs {gs}")
+    y = ops.gemv(xd, Wd, sd).cpu().double()
+    assert bool(((y - ref).abs() <= tol).all())
+    acc = base.to(dev)
+    ops.gemv(xd, Wd, sd, out=acc, epilogue="add")
+    assert bool(((acc.cpu().double() - base.double() - ref).abs() <= tol + 2.0 ** -23 * (ref.abs() + base.abs())).all())
+    a = ops.gemv(xd, Wd, sd, epilogue="swiglu", prenorm=(None, nwd, 1e-6, None)).cpu().double()
+    gate, up = refn[:, 0::2], refn[:, 1::2]
+    act = torch.nn.functional.silu(gate)
+    bound = 1.1 * toln[:, 0::2] * (up.abs() + toln[:, 1::2]) + act.abs() * toln[:, 1::2] + 2.0 ** -20 * (act * up).abs()
+    assert bool(((a - act * up).abs() <= bound).all())
+    slots, out = torch.zeros(M, dtype=torch.int64, device=dev), torch.full((M, N), float("nan"), device=dev)
+    idx = torch.empty(M, dtype=torch.int32, device=dev)
+    ops.gemv_norm_argmax(xd, Wd, sd, (None, nwd, 1e-6, None), slots, out=out, idx=idx)
+    assert bool(((out.cpu().double() - refn).abs() <= toln).all())
+    assert torch.equal(idx.long(), out.argmax(-1))
