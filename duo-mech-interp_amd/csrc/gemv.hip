@@ -512,16 +512,15 @@ __global__ __launch_bounds__(256) void swiglu_push_kernel(const float* __restric
 using q35::GemvArgs;
 
 namespace {
+constexpr int64_t kGemvCus = 256;  // compute units of the MI355X
 // Blocks of 16 output rows at which a product is split over K: below this many, an accumulating product without the
-// norm splits its K steps so that blocks x splits reaches it (one block per CU of the MI355X).
-constexpr int64_t kGemvSplitTarget = 256;
-// Rows of x from which an int8 product runs on the matrix core: the times on both sides of the line are in gemv_mfma.hip.
-constexpr int64_t kGemvMfmaRows = 4;
-// Whether an int8 product of 1 to 3 rows of x with more tiles than kGemvMaxBlocks runs the tile loop of gemv_mfma.hip (its
-// waves take whole tiles) rather than the one of this file (blocks take tiles). That one's time hardly grows with the
-// rows of x, but its 2048 waves (two blocks of four per CU) take ceil(tiles / 2048) tiles each, so a last round with few
-// tiles costs a full one, and it is slow over long rows of W; this one's blocks share a tile's K steps, and each ends on
-// an argmax atomic per row. A product and its argmax form run the same kernel, so that they give the same bits. Measured
+// norm splits its K steps so that blocks x splits reaches it (one block per CU).
+constexpr int64_t kGemvSplitTarget = kGemvCus;
+// Whether an int8 product with more tiles than kGemvMaxBlocks runs the tile loop of gemv_mfma.hip (its waves take whole
+// tiles) rather than the one of this file (blocks take tiles). That one's time hardly grows with the rows of x, but its
+// 2048 waves (two blocks of four per CU) take ceil(tiles / 2048) tiles each, so a last round with few tiles costs a full
+// one, and it is slow over long rows of W; this one's blocks share a tile's K steps, and each ends on an argmax atomic per
+// row. A product and its argmax form run the same kernel, so that they give the same bits. Measured
 // on MI355X, group scales, us, here / there, plain or behind the norm (in parentheses with norm and argmax):
 //   1 row: 151,936 x 1024 31.5 / 35.2 (34.5 / 38.8), 65,536 x 1024 16.4 / 18.1 (22.0 / 21.6), 16,400 x 1024 6.2 / 8.4 (16.1 /
 //     12.2), 32,768 x 2048 15.6 / 17.8 (23.8 / 22.0), 20,480 x 4096 20.5 / 27.6 (26.2 / 31.5); with one K step per tile
@@ -530,7 +529,12 @@ constexpr int64_t kGemvMfmaRows = 4;
 //     (23.4 / 21.6), 40,008 (61 %) 12.2 / 14.3 (17.3 / 16.2), 16,400 (50 %) 7.1 / 8.5 (17.2 / 11.6), 50,000 x 3072 (76 %) 36.0 /
 //     41.0 (39.7 / 42.6);
 //   3 rows: 151,936 x 1024 40.5 / 35.3 (44.4 / 39.0), 65,536 20.7 / 17.4, 20,480 (62 %) 9.3 / 10.5 (14.6 / 13.3); 20,480 x
-//     4096 25.4 / 44.3, where the pieces of x leave one block per CU there.
+//     4096 25.4 / 44.3, where the pieces of x leave one block per CU there;
+//   4 rows: 16,400 x 1024 9.7 / 9.1, 20,480 x 2560 29.2 / 23.2; one block per CU: 20,480 x 4096 39.9 / 52.1, 65,536 x 4096
+//     82.1 / 91.7 (behind the norm 79.3 / 81.7);
+//   6 to 8 rows (8-row tiles here; 8 rows): 151,936 x 1024 75.1 / 42.3; one block per CU: 20,480 x 2048 25.3 / 32.5, 65,536 x
+//     2048 67.4 / 56.4, behind the norm 29.9 / 29.5 and 70.3 / 50.7. 5 rows (one MFMA per fragment there, 8-row tiles here):
+//     there at every size.
 static bool gemv_tiles_on_mfma(int64_t M, int64_t K, int64_t ntiles, bool norm) {
   using namespace q35;
   const bool two = 2 * gemv_mfma_lds(4, M, K) <= kGemvLds;
@@ -538,8 +542,29 @@ static bool gemv_tiles_on_mfma(int64_t M, int64_t K, int64_t ntiles, bool norm) 
   switch (M) {
     case 1: return K < 512 && 10 * ntiles >= 9 * room;
     case 2: return two && (norm || (K <= 2048 && 10 * ntiles >= 9 * room));
-    default: return two && (norm || K < 1024 || 10 * ntiles >= 7 * room);
+    case 3: return two && (norm || K < 1024 || 10 * ntiles >= 7 * room);
+    case 4: return two;
+    case 5: return true;
+    default: return two || norm || ntiles >= waves;
   }
+}
+
+// Whether an int8 product of one tile per block runs on the matrix core (gemv_mfma.hip): from 4 rows of x (the times on
+// both sides of that line are there), except that its pieces of x take 1.5 times the LDS of the rows themselves: where
+// the blocks are not all resident at once and fewer than 16 waves fit a CU, the form of this file is the faster one.
+// Measured on MI355X, group scales, store, us, here / there:
+//   4 rows: 12,288 x 1024 (768 blocks, three per CU) 7.8 / 7.5, 12,544 x 1024 8.7 / 9.7, 16,384 x 1024 9.0 / 10.1, 16,384 x
+//     1536 (two of 8 waves) 13.4 / 12.9, 4096 x 2048 (256 blocks, one per CU) 6.3 / 6.1, 4352 x 2048 7.8 / 9.8, 12,288 x 2048
+//     13.3 / 16.1, 12,288 x 4096 22.4 / 26.7;
+//   8 rows (8-row tiles here): 8192 x 1024 (two per CU) 8.2 / 7.5, 8224 x 1024 8.7 / 11.0, 4352 x 2048 11.2 / 12.8; behind
+//     the norm the two are equal or that one is faster: 8224 x 1024 11.1 / 11.3, 4352 x 2048 with the conv 16.0 / 12.9;
+//   5 rows: 16,384 x 1024 12.3 / 10.8, 12,288 x 2048 18.5 / 16.9.
+static bool gemv_block_on_mfma(int64_t M, int64_t K, int64_t blocks, int nw, bool norm) {
+  using namespace q35;
+  if (M < 4) return false;
+  if (M == 5 || (M > 5 && norm)) return true;
+  const int64_t per_cu = kGemvLds / gemv_mfma_lds(nw, M, K);
+  return blocks <= kGemvCus * per_cu || per_cu * nw >= 16;
 }
 
 template <typename TW, int EPI, int U, bool NORM, bool GS, bool GN, int R = 4>
@@ -555,10 +580,8 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
   constexpr int R8 = R > 2 ? 2 : R;
   const int re = mp == 8 ? R8 : R;
   const int64_t ntiles = (N + 4 * re - 1) / (4 * re);
-  // kFew: int8 products of kGemvMfmaRows rows or more run gemv_mfma.hip; the 4-row tiles (R 1) stay here for every M.
   // The tile loop is compiled for every form that can have more tiles than blocks (the conv epilogue's entry point and
   // the 4-row tiles' launcher bound N), and the grid is capped only with it.
-  constexpr bool kFew = sizeof(TW) == 1 && R > 1;
   constexpr bool kLoop = EPI != kEpiConv && R > 1;
   const bool loop = kLoop && ntiles > kGemvMaxBlocks;
   const dim3 grid((unsigned)(loop ? kGemvMaxBlocks : ntiles), (unsigned)nsplit), block(64 * nw);
@@ -572,8 +595,8 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
         case 1: Q35_GEMV(1, true); break;
         case 2: Q35_GEMV(2, true); break;
         case 3: Q35_GEMV(3, true); break;
-        case 4: if constexpr (!kFew) Q35_GEMV(4, true); break;
-        default: if constexpr (!kFew && U <= 2) Q35_GEMV(8, true); break;  // 8 rows: U <= 2 (gemv_launch)
+        case 4: Q35_GEMV(4, true); break;
+        default: if constexpr (U <= 2) Q35_GEMV(8, true); break;  // 8 rows: U <= 2 (gemv_launch)
       }
       return;
     }
@@ -583,8 +606,8 @@ void gemv_launch_u(const float* x, int64_t ldx, const TW* W, const float* wscale
     case 1: Q35_GEMV(1, false); break;
     case 2: Q35_GEMV(2, false); break;
     case 3: Q35_GEMV(3, false); break;
-    case 4: if constexpr (!kFew) Q35_GEMV(4, false); break;
-    default: if constexpr (!kFew && U <= 2) Q35_GEMV(8, false); break;  // 8 rows: U <= 2 (gemv_launch)
+    case 4: Q35_GEMV(4, false); break;
+    default: if constexpr (U <= 2) Q35_GEMV(8, false); break;  // 8 rows: U <= 2 (gemv_launch)
   }
 #undef Q35_GEMV
 }
@@ -624,8 +647,8 @@ int gemv_launch(const float* x, int64_t ldx, const TW* W, const float* wscale, f
   const int nw = bsteps <= 4 ? 4 : 8;
   const int64_t per_wave = (bsteps + nw - 1) / nw;
   if constexpr (sizeof(TW) == 1) {
-    if (M >= kGemvMfmaRows || (EPI != kEpiConv && !GN && nsplit == 1 && nblk > kGemvMaxBlocks &&
-                               gemv_tiles_on_mfma(M, K, nblk, NORM)))
+    const bool tiles = EPI != kEpiConv && !GN && nsplit == 1 && nblk > kGemvMaxBlocks;
+    if (tiles ? gemv_tiles_on_mfma(M, K, nblk, NORM) : gemv_block_on_mfma(M, bsteps * 256, nblk * nsplit, nw, NORM))
       return gemv_mfma_run(NORM, GN, GS, EPI, x, ldx, W, wscale, y, ldy, M, N, K, pushes, npush, T, (int)nsplit, na, st);
   }
   // more than 4 rows of x: at most two K steps per wave in flight (four spill the registers of 8 rows)

@@ -404,13 +404,18 @@ def test_gemv_gated_norm_many_tiles(M, N, K, gs):
         assert bool((err <= bound + 2.0 ** -24 * exp.abs()).all()), f"{epi}: {int((~(err <= bound)).sum())} outputs off"
 
 
-# int8 products past 1024 tiles at 1 to 3 rows, on both sides of the line between the two tile loops: half of a round of
-# waves (16,400 rows of W), all of one (32,762, ragged), short and long rows of W, and 4096 inputs, where three rows leave one
-# block per CU
-@pytest.mark.parametrize("M", [1, 2, 3])
-@pytest.mark.parametrize("N,K", [(16400, 256), (16400, 1024), (32762, 256), (32762, 1024), (16390, 4096)])
+# int8 products on both sides of the lines between the FMA and the matrix-core forms. Past 1024 tiles: half of a round of
+# waves (16,400 rows of W), all of one (32,762, ragged), short and long rows of W, and where the rows of x leave one block
+# per CU. One tile per block: the last product whose blocks are all resident and the first past it, at one to three blocks
+# per CU.
+@pytest.mark.parametrize("M,N,K", [(m, n, k) for m in (1, 2, 3) for n, k in
+                                   [(16400, 256), (16400, 1024), (32762, 256), (32762, 1024), (16390, 4096)]] +
+                                  [(4, 16400, 2560), (4, 16390, 3072), (5, 16390, 2048), (6, 16390, 1536),
+                                   (8, 16390, 2048), (7, 32770, 2048), (4, 12288, 1024), (4, 12302, 1024),
+                                   (4, 12302, 1536), (4, 4096, 2048), (4, 4110, 2048), (4, 4110, 4096),
+                                   (5, 4110, 2048), (6, 8192, 1024), (8, 8206, 1024), (7, 4110, 2048)])
 @pytest.mark.parametrize("gs", [True, False])
-def test_gemv_tile_loops(M, N, K, gs):
+def test_gemv_both_forms(M, N, K, gs):
     """Store, accumulate, SwiGLU behind the norm and the argmax form against fp64: every output within K 2^-24 of its
     row's sum |x w| (fp32 sums; 16 roundings more for the norm and the silu, whose slope is under 1.1)."""
     dev = device()
@@ -423,7 +428,7 @@ def test_gemv_tile_loops(M, N, K, gs):
     ref, tol = x.double() @ wd.T, eps * (x.double().abs() @ wd.abs().T)
     refn, toln = h @ wd.T, eps * (h.abs() @ wd.abs().T)
     Wd, sd, xd, nwd = W.to(dev), s.to(dev), x.to(dev), nw.to(dev)
-    announce(f"gemv tile loops M{M} N{N} K{K} gs {gs}")
+    announce(f"gemv both forms M{M} N{N} K{K} gs {gs}")
     y = ops.gemv(xd, Wd, sd).cpu().double()
     assert bool(((y - ref).abs() <= tol).all())
     acc = base.to(dev)
