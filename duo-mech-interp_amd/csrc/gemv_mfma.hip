@@ -1,7 +1,7 @@
-// The decode GEMV on the matrix core (M <= 8 rows of x, int8 weights): the products, prologues and epilogues of gemv.hip,
+// The decode GEMV on the matrix core (4 to 8 rows of x, with the tile loop 1 to 8, int8 weights): the products, prologues and epilogues of gemv.hip,
 // whose launcher decides which form runs.
 //
-// The fp32 form spends one FMA per weight and row of x and reads x from LDS for every few rows of W; past three rows of x
+// The form of gemv.hip spends one FMA per weight and row of x and reads x from LDS for every few rows of W; past three rows of x
 // that sets its time, not the weights' bytes. Here x is split into three bf16 pieces, hi + mid + lo = x exactly (8
 // significant bits each, by truncation), int8 weights are exact in bf16, and a v_mfma_f32_16x16x32_bf16 multiplies 16
 // output rows by 16 columns = (piece, row of x): every product is exact and is summed in fp32, where an fp32 FMA chain
@@ -9,10 +9,11 @@
 // fit one MFMA, eight take two. Weights come in as there (a wave load covers 4 rows x 256 contiguous bytes: fragment-order
 // loads would touch another cache line with every lane), go through a 4 KB wave-private LDS tile (16-byte chunks
 // XOR-swizzled by row: no bank conflicts) and become A fragments.
-// Measured on MI355X (graph-replayed, weights past the L2; us at 4 / 5 / 8 rows of x): gate/up 7168 x 1024 with SwiGLU
-// 6.5 / 6.7 / 8.5 (fp32 form 7.6 / 15.5 / 15.7, at 8-row tiles past 4 rows), 5120 x 1024 5.7 / 6.0 / 8.4 (6.8 / 12.7 /
-// 13.0), 1024 x 2048 accumulating 4.2 / 4.6 / 5.2 (4.5 / 5.3 / 5.5). At 3 rows the two are equal (gate/up 7.2 and 6.9
-// before the changes both forms share), below that the fp32 form is faster (1 row 6.4 and 5.3).
+// Measured on MI355X (graph-replayed, weights past the L2, group scales; us at 4 / 5 / 8 rows of x): gate/up 7168 x 1024 with
+// norm and SwiGLU 6.3 / 6.4 / 7.7 (the FMA form of gemv.hip 6.7 / 9.8 / 10.0, at 8-row tiles past 4 rows), 5120 x 1024 with
+// the norm 5.7 / 5.9 / 7.9 (5.9 / 7.7 / 7.9), 1024 x 2048 accumulating 4.2 / 4.6 / 5.2 (4.4 / 5.1 / 5.2). At 3 rows the two
+// were equal (gate/up 7.2 and 6.9), at one row the FMA form was faster (6.4 and 5.3); kernels for fewer than 4 rows exist
+// only with the tile loop.
 #include <type_traits>
 
 #include "gemv_common.h"
@@ -583,7 +584,7 @@ __global__ __launch_bounds__(256, 2) void gemv_tiles_kernel(const float* __restr
   }
 }
 
-// the matrix-core form (int8 weights, one 16-row tile per block)
+// the matrix-core form (int8 weights, one 16-row tile per block; 4 rows of x or more)
 template <int EPI, int U, bool NORM, bool GS, bool GN>
 void gemv_mfma_launch_u(const float* x, int64_t ldx, const int8_t* W, const float* wscale, float* y, int64_t ldy,
                         int64_t M, int64_t N, int64_t K, const q35_push* pushes, int npush, int64_t T, int nw,
@@ -595,9 +596,6 @@ void gemv_mfma_launch_u(const float* x, int64_t ldx, const int8_t* W, const floa
   hipLaunchKernelGGL((gemv_mfma_kernel<MP, EPI, U, NORM, GS, GN>), grid, block, lds, st, x, ldx, W, wscale, y, ldy, \
                      (int)M, (int)N, (int)K, pushes, npush, (int)T, na.xadd, na.nw, na.eps, na.xout, na.aux)
   switch (gemv_mfma_rows(M)) {
-    case 1: Q35_GEMV_MFMA(1); break;
-    case 2: Q35_GEMV_MFMA(2); break;
-    case 3: Q35_GEMV_MFMA(3); break;
     case 4: Q35_GEMV_MFMA(4); break;
     case 5: Q35_GEMV_MFMA(5); break;
     default: Q35_GEMV_MFMA(8); break;
