@@ -463,9 +463,12 @@ static double pf_dispatch_time(int nqb, int Ls, bool paired, int64_t n_other, in
 // The schedule of a launch on a device of cus CUs: 0 whole blocks, longest first; 1 the long blocks in halves (Ls); 2 key
 // runs. Halves: the split schedule's estimated end plus the merge kernel (1 for its launch, 0.04 per pair of halves of
 // four waves: the partials' stores and reads). The costs were fitted to same-box timings of both schedules over ten
-// shapes (B 1-4, T 1536-8192, 8 q / 2 kv heads), whose faster schedule they all pick. Key runs: the longest run, 2 for
-// prologue and partial, and 0.04 per partial of four waves, against 1.25 times the halves' estimate, which is short for the
-// blocks under 40 tiles that have this option (fitted to B 1-3, T 300-2896). Decisions are kept per shape.
+// shapes (B 1-4, T 1536-8192, 8 q / 2 kv heads), whose faster schedule they all pick. Where key runs are an option (every
+// whole block has a CU to itself): the longest run, 5 for prologue, partial and merge, and 0.012 per partial of four waves,
+// against the whole blocks and 1.25 times the halves' estimate, which is short for these. Fitted to all three schedules
+// over 257 shapes (B 1-4, T 460-4064, 8 / 2, 8 / 1, 4 / 4 and 16 / 2 heads): 0.3 % over the best one on average, none 2.5 %
+// over. Lower costs for the runs chose them for three rows of 462 / 1200 / 1300 tokens (39.2 / 64.1 / 68.6 us, whole 34.9 /
+// 60.4 / 64.2), and halves for two rows of 600 (48.4, whole 39.2). Decisions are kept per shape.
 static int pf_schedule(int nqb, int Ls, int ks_per, int64_t n_other, int gw, int cus) {
   if (Ls == 0 && ks_per == 0) return 0;
   if (cus <= 0) return Ls ? 1 : 0;
@@ -489,22 +492,23 @@ static int pf_schedule(int nqb, int Ls, int ks_per, int64_t n_other, int gw, int
   }
   double best = pf_dispatch_time(nqb, 0, false, n_other, cus);
   int pick = 0;
+  const bool ks = ks_per && cus >= kKsSlots;
   if (Ls) {
     const bool paired = (int64_t)pf_items(nqb, Ls, true) * n_other <= cus;
-    const double split = pf_dispatch_time(nqb, Ls, paired, n_other, cus) + 1.0 + 0.01 * gw * (double)(nsq * n_other);
+    double split = pf_dispatch_time(nqb, Ls, paired, n_other, cus) + 1.0 + 0.01 * gw * (double)(nsq * n_other);
+    if (ks) split *= 1.25;
     if (split < best) {
       best = split;
       pick = 1;
     }
   }
-  if (ks_per && cus >= kKsSlots) {
-    if (pick == 1) best *= 1.25;
+  if (ks) {
     int64_t parts = 0;
     for (int qb = 0; qb < nqb; ++qb) {
       const int n = (pf_tiles(qb) + ks_per - 1) / ks_per;
       parts += n > 1 ? n : 0;
     }
-    if (ks_per + 2.0 + 0.01 * gw * (double)(parts * n_other) < best) pick = 2;
+    if (ks_per + 5.0 + 0.003 * gw * (double)(parts * n_other) < best) pick = 2;
   }
   std::lock_guard<std::mutex> lock(mu);
   keys[next] = Key{nqb, gw, cus, ks_per, n_other};
