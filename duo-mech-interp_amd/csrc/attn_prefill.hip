@@ -20,7 +20,6 @@
 // online softmax in registers, then O^T += V^T P^T with P^T's accumulator tiles used directly as B operands. Tiles
 // arrive by global_load_lds DMA into XOR-swizzled LDS (conflict-free 16-byte operand reads), two stages and one
 // barrier per tile (tile kt + 1 is copied while tile kt is computed), each wave copying a quarter of every tile.
-#include <atomic>
 #include <functional>
 #include <mutex>
 #include <queue>
@@ -420,22 +419,26 @@ __device__ inline int pf_nkt(bool cached, int qb, int qshift, int T) {
 }
 
 // The own-keys form's run length: the shortest whose runs fit `slots` blocks at once; 0: none, or one run per block.
-// *ns: the most runs of a block.
+// *ns: the most runs of a block. Longer runs are never more, so the shortest is found by halving (a call searches twice,
+// in the workspace's size and the launch: length by length a search took 2 to 5 us at 3000 to 4000 tokens on one row).
 inline int pf_ks_len(int nqb, int64_t n_other, int slots, int* ns) {
   if ((int64_t)nqb * n_other >= slots) return 0;
   const int nmax = pf_tiles(nqb - 1);
   if (nmax < 2 * kKsMinTiles) return 0;
-  int64_t tiles = 0;
-  for (int qb = 0; qb < nqb; ++qb) tiles += pf_tiles(qb);
-  const int64_t least = (tiles * n_other + slots - 1) / slots;
-  for (int per = least > kKsMinTiles ? (int)least : kKsMinTiles; per < nmax; ++per) {
+  auto fits = [&](int per) {
     int64_t runs = 0;
-    for (int qb = 0; qb < nqb && runs * n_other <= slots; ++qb)
-      runs += (pf_tiles(qb) + per - 1) / per;
-    *ns = (nmax + per - 1) / per;
-    if (runs * n_other <= slots && (int64_t)nqb * n_other * *ns <= 2 * (int64_t)slots) return per;
+    for (int qb = 0; qb < nqb; ++qb) runs += (pf_tiles(qb) + per - 1) / per;
+    return runs * n_other <= slots && (int64_t)nqb * n_other * ((nmax + per - 1) / per) <= 2 * (int64_t)slots;
+  };
+  int lo = kKsMinTiles, hi = nmax;  // (runs of nmax tiles: whole blocks, which fit)
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (fits(mid)) hi = mid;
+    else lo = mid + 1;
   }
-  return 0;
+  if (lo >= nmax) return 0;
+  *ns = (nmax + lo - 1) / lo;
+  return lo;
 }
 constexpr int kKsSlots = 256;  // the blocks that the workspace holds runs for (one per CU of the MI355X), twice over
 
@@ -1081,19 +1084,6 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_runs_kernel(const floa
 
 static int64_t padded_T(int64_t T) { return (T + kBN - 1) / kBN * kBN; }
 
-// Compute units of the current device, queried once per device (the paired work order needs every block resident).
-static int device_cus() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 // Workspace: K rotated and V transposed ([B, Hkv, Tp, D] bf16 each), for the projection-output form the rotated
 // queries ([B, T, Hq, D] bf16), then the partials of the split blocks ([pairs][2 halves][wave] x kPartFloats fp32) or of the
 // key runs ([query block and (row, kv head, group)][NS runs][wave]).
@@ -1102,12 +1092,13 @@ struct PfLayout {
   int64_t npairs;
   int ks_per, ks_ns;  // key runs: the shortest run, the most runs of a query block (0: not an option)
 };
-// Ls: the split length (the workspace functions size for pf_split_len, the most a launch can use).
-static PfLayout pf_layout(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, bool fp, int Ls) {
+// Sized for halves of pf_split_len tiles, the most a launch can use.
+static PfLayout pf_layout(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, bool fp) {
   const int64_t Tp = padded_T(T);
   const int64_t G = Hq / Hkv;
   const int64_t GW = G > 4 ? 4 : G;
   const int64_t nqb = (T + kBQ - 1) / kBQ;
+  const int Ls = pf_split_len((int)nqb);
   const int64_t nsq = Ls ? nqb - 2 * Ls : 0;
   PfLayout l;
   l.npairs = nsq * B * Hkv * (G / GW);
@@ -1152,7 +1143,7 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
   const int64_t n_other = B * Hkv * ngroups;
   if ((int64_t)pf_items((int)nqb, Lmax, false) * n_other > 0x7fffffff) return Q35_EUNSUPPORTED;
   // the workspace, checked before any HIP call: the split case's, or as the size functions report it with room for runs
-  const PfLayout lay0 = pf_layout(B, T, Hq, Hkv, FP, Lmax);
+  const PfLayout lay0 = pf_layout(B, T, Hq, Hkv, FP);
   if (lay0.npairs > 0x7fffffff) return Q35_EUNSUPPORTED;
   if (!workspace || workspace_bytes < lay0.base || ((uintptr_t)workspace & 255)) return Q35_EWORKSPACE;
   // the first HIP call: the device's compute units decide the split and the work order
@@ -1160,16 +1151,16 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
   const int sched = pf_schedule((int)nqb, Lmax, workspace_bytes < lay0.total ? 0 : lay0.ks_per, n_other, GW, cus);
   const bool runs = sched == 2;
   const int Ls = sched == 1 ? Lmax : 0;
-  const PfLayout lay = pf_layout(B, T, Hq, Hkv, FP, Ls);
+  const int64_t npairs = Ls ? lay0.npairs : 0;
   const bool paired = Ls > 0 && (int64_t)pf_items((int)nqb, Ls, true) * n_other <= cus;
-  const int64_t nblocks = runs ? (int64_t)nqb * lay.ks_ns * n_other : (int64_t)pf_items((int)nqb, Ls, paired) * n_other;
+  const int64_t nblocks = runs ? (int64_t)nqb * lay0.ks_ns * n_other : (int64_t)pf_items((int)nqb, Ls, paired) * n_other;
   char* ws = static_cast<char*>(workspace);
   __bf16* kr = reinterpret_cast<__bf16*>(ws);
   __bf16* vt = kr + (size_t)B * Hkv * Tp * kPD;
-  float* part = reinterpret_cast<float*>(ws + lay.part_off);
+  float* part = reinterpret_cast<float*>(ws + lay0.part_off);
   PfFront fe = fe0;
   if constexpr (FP) {
-    fe.qr = reinterpret_cast<__bf16*>(ws + lay.q_off);
+    fe.qr = reinterpret_cast<__bf16*>(ws + lay0.q_off);
     q = fe.qr;
   }
   const dim3 gp((unsigned)((FP ? 2 + G : 2) * (Tp / kBN)), (unsigned)Hkv, (unsigned)B);
@@ -1191,13 +1182,13 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
                            : paired ? attn_prefill_kernel<GG, true, FP, false> : attn_prefill_kernel<GG, false, FP, false>), \
                      dim3((unsigned)nblocks), dim3(64 * GG), 0, st, (const __bf16*)q, kr, vt, gate, gate_ld, cos, sin, \
                      (int)pos0, (__bf16*)out, (int)T, (int)Tp, (int)Hq, (int)Hkv, ngroups, mrot, scale, (int)nqb,     \
-                     (int)B, runs ? lay.ks_per : Ls, lay.ks_ns, part, (const int32_t*)nullptr);                     \
+                     (int)B, runs ? lay0.ks_per : Ls, lay0.ks_ns, part, (const int32_t*)nullptr);                     \
   if (runs)                                                                                                         \
     hipLaunchKernelGGL((attn_prefill_merge_runs_kernel<GG, FP>), dim3((unsigned)(nqb * n_other), GG), dim3(256), 0, st, \
                        part, gate, gate_ld, (__bf16*)out, (int)T, (int)Tp, (int)Hq, (int)Hkv, ngroups, (int)B,       \
-                       lay.ks_per, lay.ks_ns, (const int32_t*)nullptr);                                             \
-  else if (lay.npairs > 0)                                                                                          \
-    hipLaunchKernelGGL((attn_prefill_merge_kernel<GG, FP>), dim3((unsigned)lay.npairs, GG), dim3(256), 0, st, part,  \
+                       lay0.ks_per, lay0.ks_ns, (const int32_t*)nullptr);                                             \
+  else if (npairs > 0)                                                                                              \
+    hipLaunchKernelGGL((attn_prefill_merge_kernel<GG, FP>), dim3((unsigned)npairs, GG), dim3(256), 0, st, part,  \
                        gate, gate_ld, (__bf16*)out, (int)T, (int)Hq, (int)Hkv, ngroups, (int)B, Ls)
   switch (GW) {
     case 1: Q35_PF_LAUNCH(1); break;
@@ -1213,7 +1204,7 @@ static int pf_launch(const void* q, const void* k, const void* v, const void* ga
 extern "C" size_t q35_gated_attn_prefill_workspace_bytes(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t D) {
   using namespace q35;
   if (pf_check(B, T, Hq, Hkv, D, 0) != Q35_OK) return 0;
-  return pf_layout(B, T, Hq, Hkv, false, pf_split_len((int)((T + kBQ - 1) / kBQ))).total;
+  return pf_layout(B, T, Hq, Hkv, false).total;
 }
 
 extern "C" int q35_gated_attn_prefill(const void* q, const void* k, const void* v, const void* gate,
@@ -1233,7 +1224,7 @@ extern "C" size_t q35_gated_attn_prefill_proj_workspace_bytes(int64_t B, int64_t
                                                               int64_t D) {
   using namespace q35;
   if (pf_check(B, T, Hq, Hkv, D, 0) != Q35_OK) return 0;
-  return pf_layout(B, T, Hq, Hkv, true, pf_split_len((int)((T + kBQ - 1) / kBQ))).total;
+  return pf_layout(B, T, Hq, Hkv, true).total;
 }
 
 extern "C" int q35_gated_attn_prefill_proj(const float* y, int64_t ldy, const float* q_norm_w,

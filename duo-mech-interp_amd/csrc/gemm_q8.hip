@@ -888,11 +888,8 @@ static int gemm_few_launch(const float* x, int64_t ldx, const int8_t* W, const f
 
 // compute units of the current device (the DMA kernel runs one block per CU)
 static int64_t gemm_cu_count() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
+  const int cus = device_cus();
+  return cus > 0 ? cus : 256;
 }
 
 // The few-row kernel's tile for a product, 0 where the tiled kernels are faster. `wide`: the DMA kernel would run it.

@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
@@ -57,6 +59,20 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 #define Q35_ARGS_UPFRONT(...) asm volatile("" ::Q35_FOR_EACH(Q35_SGPR_OPERAND, __VA_ARGS__))
 
 namespace q35 {
+
+// Compute units of the current device, asked of the runtime once per device; 0 if it cannot tell. Launchers size grids and
+// choose schedules by it.
+inline int device_cus() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 0;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
 
 // Element types the kernels accept for activations (q, k, v, o, gate).
 enum DType : int { kF32 = 0, kBF16 = 1 };
