@@ -398,8 +398,8 @@ inline int pf_items(int nqb, int Ls, bool paired) {
 // 2500 tokens 31.5 / 41.2 / 54.2 / 67.3 against 41.8 / 52.3 / 70.2 / 80.2, two rows of 1000 44.8 / 54.5, three rows of
 // 1000 51.5 / 58.7; over the cache (front end included), 2 tokens at 1700 keys 26.3 / 63.8, at 7000 39.7 / 217; three rows
 // of 128 tokens at 1700 keys 40.2 / 77.0. Runs of at least 4 tiles: a partial and its share of the merge cost about half
-// a tile. A cache of under 12 tiles is not cut (5 tiles as 4 + 1: 30.9 against 27.9); a short context in a longer cache
-// pays the merge's launch, 1.7 us of 20-30, since its length is on the device.
+// a tile. Over the cache the rows whose keys end under pf_row_cuts' line stay whole, and a cache of under 12 tiles is never
+// cut; a short context in a longer cache still pays the merge's launch, 1.6 us of 16-30, since its length is on the device.
 constexpr int kKsMinTiles = 4;
 
 struct PfRun {
@@ -417,6 +417,12 @@ __host__ __device__ inline PfRun pf_run(int nkt, int full, int min_per, int NS, 
 __device__ inline int pf_nkt(bool cached, int qb, int qshift, int T) {
   return cached ? (qshift + min(qb * kBQ + kBQ - 1, T - 1)) / kBN + 1 : pf_tiles(qb);
 }
+
+// Whether the query blocks of a row of T tokens at position qshift of the cache are cut: from 7 key tiles for up to 64
+// tokens, from 9 for more (three rows, us, before key runs / cut: 200 tokens after 64, 5 tiles, 29.0 / 34.2; 128 after 200,
+// 6 tiles, 32.2 / 35.7; 200 after 200, 7 tiles, 35.4 / 37.7; 33 after 400, 7 tiles, 31.5 / 27.5; 64 after 400, 8 tiles, 34.3 /
+// 29.5; 128 after 400, 9 tiles, 38.1 / 34.2).
+__device__ inline bool pf_row_cuts(int qshift, int T) { return (qshift + T - 1) / kBN + 1 >= (T <= 64 ? 7 : 9); }
 
 // The own-keys form's run length: the shortest whose runs fit `slots` blocks at once; 0: none, or one run per block.
 // *ns: the most runs of a block. Longer runs are never more, so the shortest is found by halving (a call searches twice,
@@ -598,7 +604,8 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
     const int qb = it.qb;
     const int q0 = qb * kBQ;
     if constexpr (KS) {
-      const PfRun r = pf_run(pf_nkt(pos_dev != nullptr, qb, qshift, T), (qshift + q0) / kBN, Ls, NS, it.half);
+      const int nkt = pf_nkt(pos_dev != nullptr, qb, qshift, T);
+      const PfRun r = pf_run(nkt, (qshift + q0) / kBN, pos_dev && !pf_row_cuts(qshift, T) ? nkt : Ls, NS, it.half);
       if (it.half >= r.n) return;
       it.kt0 = r.kt0;
       it.kt1 = r.kt1;
@@ -1012,6 +1019,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_runs_kernel(const floa
   const int b = rem / (Hkv * ngroups), kvh = (rem / ngroups) % Hkv, hg = rem % ngroups;
   const int h = kvh * (Hq / Hkv) + hg * GW + wave;
   const int qshift = pos_dev ? min(max(pos_dev[b], 0), Tp - T) : 0;
+  if (pos_dev && !pf_row_cuts(qshift, T)) return;
   const int n = pf_run(pf_nkt(pos_dev != nullptr, qb, qshift, T), (qshift + qb * kBQ) / kBN, min_per, NS, 0).n;
   if (n == 1) return;
   const int l = tid & 63, tq = qb * kBQ + (l & 31);  // every chunk of thread t has lane l = t & 63

@@ -238,7 +238,10 @@ def test_attn_prefill_from_projection(B, T, Hq, Hkv, pos0, max_len):
                                                      # long caches: key runs, on rows of one run and of many, runs that
                                                      # end on the call's first tile, GQA 8 (two groups) and 1
                                                      (3, 100, 8, 2, 2304, [0, 1000, 2204]), (1, 2, 8, 2, 1024, [63]),
-                                                     (2, 33, 16, 2, 1024, [64, 991]), (1, 128, 4, 4, 768, [640])])
+                                                     (2, 33, 16, 2, 1024, [64, 991]), (1, 128, 4, 4, 768, [640]),
+                                                     # rows on both sides of the lines under which a row stays whole
+                                                     # (keys that end in the 7th tile, past 64 tokens in the 9th)
+                                                     (2, 64, 8, 2, 768, [320, 321]), (2, 66, 8, 2, 768, [446, 447])])
 def test_attn_prefill_over_cache_from_projection(B, T, Hq, Hkv, max_len, pos):
     """The multi-token call over the cache from the fused projection output (q35_gated_attn_prefill_cached_proj: the
     front end and the cache append in the pre-pass, whose value blocks take the earlier rows from the cache and the
