@@ -401,6 +401,9 @@ inline int pf_items(int nqb, int Ls, bool paired) {
 // a tile. Over the cache the rows whose keys end under pf_row_cuts' line stay whole, and a cache of under 12 tiles is never
 // cut; a short context in a longer cache still pays the merge's launch, 1.6 us of 16-30, since its length is on the device.
 constexpr int kKsMinTiles = 4;
+// A run's first running max. Finite, so that keys with a score of -inf (a key masked by its own values) weigh 0 wherever a
+// run begins, as they do in the middle of a block; below every finite score.
+constexpr float kKsMaxFrom = -3.0e38f;
 
 struct PfRun {
   int kt0, kt1, n;  // tiles of run s, number of runs
@@ -675,7 +678,7 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
     // Scores are kept unscaled; the softmax works in base 2 on scaled scores: p = 2^(s c - m) with c = scale log2(e),
     // m_run the running max of s c.
     const float csc = scale * 1.44269504088896341f;
-    float m_run = -INFINITY, l_run = 0.f;
+    float m_run = KS ? kKsMaxFrom : -INFINITY, l_run = 0.f;
     const int tq = q0 + ln;  // this lane's query
     const int full_tiles = (qshift + q0) / kBN;  // tiles entirely below this block's first query: no mask
 
@@ -812,7 +815,7 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
     // never leaves the MFMA accumulators there; the rescale (a read, multiply and write-back of all 128 accumulator
     // registers) sits outside it and runs a few times per block (always at tile 0). Every lane has a finite score in
     // the first tile of its item (key 0, or a split block's first key, is at or before its query), so m_run is finite
-    // from then on.
+    // from then on (a run's m_run always).
     int kt = it.kt0;
     while (kt < it.kt1) {
       f32x16 sc[2];
@@ -860,7 +863,8 @@ __global__ __launch_bounds__(64 * GW, 1) void attn_prefill_kernel(
     __syncthreads();
     char* ob = reinterpret_cast<char*>(&stage[0]) + 32768 * wave;
     {
-      const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+      // (KS: no weight at all, every score -inf, gives NaN like the softmax)
+      const float inv = KS || l_run > 0.f ? 1.f / l_run : 0.f;
 #pragma unroll
       for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
@@ -1050,7 +1054,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_runs_kernel(const floa
   float mm = -INFINITY, lt = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) o[j] = zero4();
-  auto add = [&](int i) {  // (every run's maximum is finite)
+  auto add = [&](int i) {  // (every run's maximum is finite, kKsMaxFrom where all of its scores are -inf)
     const float mn = fmaxf(mm, mw[i]);
     const float c0 = __builtin_amdgcn_exp2f(mm - mn), c1 = __builtin_amdgcn_exp2f(mw[i] - mn);
     mm = mn;
@@ -1069,7 +1073,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_runs_kernel(const floa
     add(1);
   }
   if (tq >= T) return;
-  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  const float inv = 1.f / lt;  // (every score -inf: 0 times infinity, NaN like the softmax)
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int mtc = (tid + 256 * j) >> 6, d = 8 * mtc + 4 * (l >> 5);

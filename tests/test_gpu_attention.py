@@ -65,6 +65,27 @@ def test_prefill_key_runs(B, T, Hq, Hkv):
     assert torch.equal(out, q35hip.gated_attention_prefill(*args))
 
 
+@pytest.mark.parametrize("first,last", [(256, 512), (320, 400), (0, 1)])
+def test_prefill_key_runs_with_minus_infinity_scores(first, last):
+    """Keys whose own values make their score -inf weigh nothing, also where they fill a whole run (tiles 4 to 7) or its
+    first tiles; a query with no other key (query 0 of the last case) is NaN, as the softmax of nothing but -inf."""
+    dev = device()
+    T = 1000
+    inp = workloads.attn_prefill_inputs(B=1, T=T, seed=5)
+    inp["q"][..., 200] = 1.0
+    inp["k"][..., 200] = 0.0
+    inp["k"][:, first:last, :, 200] = float("-inf")
+    cos, sin = _tables(T)
+    ref = oracle.gated_attention(inp["q"], inp["k"], inp["v"], inp["gate"], cos, sin)
+    d = workloads.to_device(inp, dev)
+    announce(f"attn prefill key runs, keys {first}..{last - 1} at -inf")
+    out = q35hip.gated_attention_prefill(d["q"], d["k"], d["v"], d["gate"], cos.to(dev), sin.to(dev)).float().cpu()
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert int(ref.isnan().any(-1).sum()) == (1 if first == 0 else 0)
+    q0 = last if first == 0 else 0
+    assert oracle.rel_err(out[:, q0:], ref[:, q0:]) <= 8e-3 and _worst_row(out[:, q0:], ref[:, q0:]) <= 2e-2
+
+
 def test_prefill_workspace_without_room_for_runs():
     """A workspace with room for K, V^T and the split halves only (T 512, 8 query / 2 kv heads: 16 pairs of halves of
     four waves) is taken, by another schedule; one byte less is refused before any launch."""
