@@ -892,7 +892,11 @@ static int64_t gemm_cu_count() {
   return cus > 0 ? cus : 256;
 }
 
-// The few-row kernel's tile for a product, 0 where the tiled kernels are faster. `wide`: the DMA kernel would run it.
+// What runs a product that the few-row kernel does not take: the register-staged kernel, the DMA kernel, or the
+// register-staged kernel for the rows that the DMA kernel leaves over.
+enum GemmElse { kElseRs, kElseDma, kElseTail };
+
+// The few-row kernel's tile for a product, 0 where the other kernel is faster.
 // Measured on MI355X (group scales, weights cycled past the L2, us; gate_up 7168 x 1024, down 1024 x 3584, gdn_in
 // 8224 x 1024, attn_in 5120 x 1024):
 //   1  32 x 32, 8 waves: one block per CU, the shortest K run per wave; best while its blocks fit one round (gate_up
@@ -902,17 +906,25 @@ static int64_t gemm_cu_count() {
 //   3  32 x 64, 4 waves, two blocks per CU: more than one round, against the DMA kernel (which takes the same time up
 //      to about 700 rows, one round of tiles). gate_up 200 / 300 / 400 / 500 rows 20.9 / 26.2 / 31.2 / 35.5 against
 //      37.6 / 37.9 / 38.4 / 38.6; gdn_in 200 / 300 / 400 rows 20.8 / 28.0 / 33.3 against 30.2 / 31.0 / 31.6; attn_in
-//      500 / 700 rows 25.6 / 34.1 against 30.5 / 31.4: the lines cross at about 1400 blocks.
+//      500 / 700 rows 25.6 / 34.1 against 30.5 / 31.4: the lines cross at about 1400 blocks. At K < 512 the waves' sums
+//      weigh more: 3072 x 256 at 640 / 768 rows 11.8 / 14.9 against 13.4 / 13.7, about 1000 blocks.
+//      Against the register-staged kernel, for the rows a wide product leaves over (store / SwiGLU): 5120 x 1024 at 256 /
+//      384 / 512 rows 19.1 / 23.2 / 28.2 against 21.1 / 21.7 / 25.7, gate_up at 256 / 384 rows 23.4 / 31.9 against 23.9 /
+//      27.6, 16,384 x 1024 at 128 rows 25.2 against 22.7, 3072 x 256 at 256 / 384 rows 7.2 / 10.1 against 7.9 / 8.1, 3072 x 512
+//      at 384 / 512 rows 12.5 / 13.5 against 12.5 / 12.9, 4096 x 2048 at 512 / 640 rows 43.8 / 53.5 against 43.3 / 49.7: 900
+//      blocks at K 1024, fewer with shorter rows.
 //   4  64 x 64, 4 waves: more than one round of tile 2, against the register-staged kernel, while its blocks fit one
-//      round (down 700 / 1000 rows 32.8 / 33.8 against 34.2 / 39.7 for tile 3 and 66.1 / 66.4).
-static int gemm_few_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int xbytes, bool wide) {
+//      round (down 700 / 1000 rows 32.8 / 33.8 against 34.2 / 39.7 for tile 3 and 66.1 / 66.4; not at K < 512, 1024 x 256
+//      at 1024 rows 8.5 against 8.0, bf16 x 7.4 against 6.5).
+static int gemm_few_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int xbytes, GemmElse other) {
   if (K > 128 * kFewGroups || ((M - 1) * ldx + K) * xbytes > 0xffffffffLL || N * K > 0xffffffffLL) return 0;
   const int64_t cus = gemm_cu_count();
   const int64_t m32 = (M + 31) / 32, n64 = (N + 63) / 64;
   if (m32 * ((N + 31) / 32) <= cus) return 1;
   if (m32 * n64 <= cus) return 2;
-  if (wide) return m32 * n64 <= 5 * cus + cus / 4 ? 3 : 0;
-  return ((M + 63) / 64) * n64 <= cus ? 4 : 0;
+  if (other == kElseDma) return 4 * m32 * n64 <= (K < 512 ? 16 : 21) * cus ? 3 : 0;
+  if (other == kElseTail) return 512 * m32 * n64 <= (768 + K < 2048 ? 768 + K : 2048) * cus ? 3 : 0;
+  return K >= 512 && ((M + 63) / 64) * n64 <= cus ? 4 : 0;
 }
 
 // a product by the few-row kernel where that is the faster one, else by the register-staged kernel
@@ -1034,7 +1046,7 @@ static int gemm_q8_run(const float* x, int64_t ldx, const int8_t* W, int w_dtype
   const bool wide =
       !XB && N >= 2048 && K <= 128 * kDGS && ((M - 1) * ldx + K) * 4 <= 0xffffffffLL && N * K <= 0xffffffffLL;
   constexpr int xb = XB ? 2 : 4, XF = XB ? 2 : XS ? 1 : 0;
-  const int tile = gemm_few_tile(M, N, K, ldx, xb, wide);
+  const int tile = gemm_few_tile(M, N, K, ldx, xb, wide ? kElseDma : kElseRs);
   if (wide && tile == 0) {
     // One block per CU, so a last round of blocks that is mostly empty costs as much as a full one. A partial last
     // column tile that costs a whole extra round (the GDN input projection: 8192 + 32 columns) runs in a
@@ -1060,13 +1072,13 @@ static int gemm_q8_run(const float* x, int64_t ldx, const int8_t* W, int w_dtype
     if (r != Q35_OK) return r;
     if (Md < M) {
       r = gemm_small_launch<XF>(x + Md * ldx, ldx, W, w_scale, y + Md * ldy, ldy, M - Md, Nd, K, epilogue, gs, pushes,
-                                npush, T, Md, ys, cap, st, gemm_few_tile(M - Md, Nd, K, ldx, xb, true));
+                                npush, T, Md, ys, cap, st, gemm_few_tile(M - Md, Nd, K, ldx, xb, kElseTail));
       if (r != Q35_OK) return r;
     }
     if (Nd < N)
       r = gemm_small_launch<XF>(x, ldx, W + Nd * K, w_scale + (gs ? Nd * (K / 128) : Nd), y + Nd, ldy, M, N - Nd, K,
                                 epilogue, gs, pushes, npush, T, 0, ys, cap, st,
-                                gemm_few_tile(M, N - Nd, K, ldx, xb, false));
+                                gemm_few_tile(M, N - Nd, K, ldx, xb, kElseRs));
     return r;
   }
   return gemm_small_launch<XF>(x, ldx, W, w_scale, y, ldy, M, N, K, epilogue, gs, pushes, npush, T, 0, ys, cap, st,

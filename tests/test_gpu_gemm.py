@@ -274,3 +274,34 @@ def test_gemm_q8_tile_order(x_form, M, N, K):
     y = ops.gemm_q8(ops.split_activations(xd) if x_form == "split" else xd, q.to(dev), s.to(dev)).cpu()
     bound = (2.0 ** -17 + 2 * K * 2.0 ** -24) * (x.double().abs() @ w.abs().T)
     assert bool(((y.double() - x.double() @ w.T).abs() <= bound).all())
+
+
+# the rows that a wide product leaves over after the DMA kernel's full rounds: 32 and 128 of 544 and 640 rows at 64 column
+# tiles (few-row, register-staged), 768 of 3072 at 12 (register-staged), and just under and at the few-row kernel's lines
+# for short K (few-row and DMA, few-row and register-staged)
+@pytest.mark.parametrize("x_form", ["fp32", "split"])
+@pytest.mark.parametrize("M,N,K", [(544, 16384, 128), (640, 16384, 128), (3072, 3072, 256), (672, 3072, 256),
+                                   (704, 3072, 256), (1024, 1024, 256)])
+def test_gemm_q8_left_over_rows(x_form, M, N, K):
+    """Store, and SwiGLU with a push per batch row, on every output against fp64: x = hi + lo drops at most 2^-17 of each
+    value and a fp32 sum of K products (the kernel's two, hi and lo) 2 K roundings of 2^-24, both of sum |x w|; the silu
+    a few roundings more at a slope under 1.1."""
+    dev = device()
+    q, s = _q8g(N, K, M + N + K)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(K + M))
+    xd = x.to(dev)
+    xin = ops.split_activations(xd) if x_form == "split" else xd
+    w = omlp.q8_dequant(q, s).double()
+    ref = x.double() @ w.T
+    tol = (2.0 ** -17 + 2 * K * 2.0 ** -24) * (x.double().abs() @ w.abs().T)
+    announce(f"gemm_q8 left-over rows {x_form} M{M} N{N} K{K}")
+    y = ops.gemm_q8(xin, q.to(dev), s.to(dev)).cpu().double()
+    assert bool(((y - ref).abs() <= tol).all())
+    T = (M + 2) // 3
+    pk = ops.pack_pushes([(3, "add", [1.0, -2.0, 0.5])], dev)
+    a = ops.gemm_q8(xin, q.to(dev), s.to(dev), epilogue="swiglu", pushes=pk, T=T).cpu().double()
+    act, up = torch.nn.functional.silu(ref[:, 0::2]), ref[:, 1::2]
+    exp = act * up
+    bound = 1.1 * tol[:, 0::2] * (up.abs() + tol[:, 1::2]) + act.abs() * tol[:, 1::2] + 2.0 ** -20 * exp.abs()
+    exp[:, 3] += torch.tensor([1.0, -2.0, 0.5]).double()[torch.arange(M) // T]
+    assert bool(((a - exp).abs() <= bound + 2.0 ** -23 * exp.abs()).all())
