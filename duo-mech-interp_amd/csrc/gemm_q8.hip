@@ -460,11 +460,12 @@ __global__ __launch_bounds__(512, 1) void gemm_q8_dma_kernel(const float* __rest
 // eight column tiles of 128 (N = 1024) put each column on its own XCD and every XCD read all of x (584 MB fetched for
 // 88 MB of x). Cold inputs, 6144 rows: 1024 x 3584 accumulating 146 -> 132 us, 1024 x 2048 88 -> 82. Few rows against a
 // wide W are the other way round: consecutive tiles read all of W into every L2, dealt ones read a column of W into one.
-// So a multiple of eight column tiles is dealt while x has less than half the bytes of W (bf16 x, group scales, us, dealt
+// So with bf16 x (the one form that comes here with a wide W and many rows) a multiple of eight column tiles is dealt, DEAL,
+// while x has less than half the bytes of W (a template: the choice inside the kernel cost 1 to 3 %; group scales, us, dealt
 // / consecutive: 256 x 16,384 x 1024 24.5 / 26.3, 256 x 7168 16.4 / 17.4, 512 x 4096 x 4096 57.8 / 62.2, 2048 x 16,384 102 /
 // 108, 3072 x 16,384 157 / 160; past the line 4096 x 16,384 231 / 218, 6144 x 2048 x 2048 96 / 88).
 // XF: x fp32 (0), in the split layout (1), or bf16 (2: hi = x exactly, lo = 0, so the lo products are skipped)
-template <int BM, int EPI, bool GS, int XF>
+template <int BM, int EPI, bool GS, int XF, bool DEAL>
 __global__ __launch_bounds__(256, 2) void gemm_q8_rs_kernel(const float* __restrict__ X, int64_t ldx,
                                                          const int8_t* __restrict__ W, const float* __restrict__ ws,
                                                          float* __restrict__ Y, int64_t ldy, int M, int N, int K,
@@ -481,11 +482,10 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_rs_kernel(const float* __restr
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int nbn = (N + kGN - 1) / kGN;
-  // tile order: dealt (see above), or as in the DMA kernel: each XCD takes consecutive tiles, n fastest inside an m panel
+  // tile order: dealt, or as in the DMA kernel: each XCD takes consecutive tiles, n fastest inside an m panel
   const int ntiles = (int)gridDim.x;
   const int xj = (int)(blockIdx.x & 7), xq = ntiles >> 3, xr = ntiles & 7;
-  const bool deal = (nbn & 7) == 0 && M < N / (XF == 2 ? 4 : 8);
-  const int tile = deal ? (int)blockIdx.x : xj * xq + min(xj, xr) + (int)(blockIdx.x >> 3);
+  const int tile = DEAL ? (int)blockIdx.x : xj * xq + min(xj, xr) + (int)(blockIdx.x >> 3);
   const int bm = tile / nbn, bn = tile - bm * nbn;
   const int m0 = bm * BM, n0 = bn * kGN;
 
@@ -970,9 +970,11 @@ static int gemm_rs_launch(const float* x, int64_t ldx, const int8_t* W, const fl
   const int BM = big ? 128 : 64;
   const int64_t nblocks = ((M + BM - 1) / BM) * nbn;
   if (nblocks > 0x7fffffff) return Q35_EUNSUPPORTED;
+  const bool deal = XF == 2 && nbn % 8 == 0 && M < N / 4;
 #define Q35_GEMM_LAUNCH(BMV, E, G)                                                                                   \
-  hipLaunchKernelGGL((gemm_q8_rs_kernel<BMV, E, G, XF>), dim3((unsigned)nblocks), dim3(256), 0, st, x, ldx, W,       \
-                     w_scale, y, ldy, (int)M, (int)N, (int)K, pushes, (int)npush, (int)T, (int)moff, ys, cap)
+  hipLaunchKernelGGL((deal ? gemm_q8_rs_kernel<BMV, E, G, XF, XF == 2> : gemm_q8_rs_kernel<BMV, E, G, XF, false>),     \
+                     dim3((unsigned)nblocks), dim3(256), 0, st, x, ldx, W, w_scale, y, ldy, (int)M, (int)N, (int)K,   \
+                     pushes, (int)npush, (int)T, (int)moff, ys, cap)
 #define Q35_GEMM_EPI(BMV, G)                                              \
   if (epilogue == kGemmStore) Q35_GEMM_LAUNCH(BMV, kGemmStore, G);        \
   else if (epilogue == kGemmAccumulate) Q35_GEMM_LAUNCH(BMV, kGemmAccumulate, G); \

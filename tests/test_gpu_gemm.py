@@ -255,11 +255,11 @@ def test_gemm_q8_few_rows(x_form, M, N, K, gs):
 
 
 # the register-staged kernel's tile orders: 297 tiles of 64 rows (8 x 37 + 1), and 8300 rows, where fp32 and split x take
-# 1170 tiles of 64 rows and bf16 x 585 of 128, each with ragged last tiles in both directions; a wide W at the last row count
-# whose tiles are dealt (bf16: N / 4, the others, past the DMA kernel's K: N / 8) and the first past it
+# 1170 tiles of 64 rows and bf16 x 585 of 128, each with ragged last tiles in both directions; a wide W, whose tiles are
+# dealt for bf16 x up to N / 4 rows (the last such row count and the first past it, with 64-row and 128-row tiles)
 @pytest.mark.parametrize("x_form", ["fp32", "split", "bf16"])
 @pytest.mark.parametrize("M,N,K", [(2085, 1050, 128), (8300, 1030, 128), (1022, 4094, 128), (1023, 4094, 128),
-                                   (510, 4094, 2176), (511, 4094, 2176)])
+                                   (510, 4094, 2176), (2047, 8192, 128), (2048, 8192, 128)])
 def test_gemm_q8_tile_order(x_form, M, N, K):
     """Every output against the fp64 product of the dequantised weights: x = hi + lo drops at most 2^-17 of each value
     and a fp32 sum of K products (the kernel's two, hi and lo) 2 K roundings of 2^-24, both of sum |x w|."""
