@@ -893,7 +893,7 @@ static int64_t gemm_cu_count() {
 }
 
 // What runs a product that the few-row kernel does not take: the register-staged kernel, the DMA kernel, or the
-// register-staged kernel for the rows that the DMA kernel leaves over.
+// register-staged kernel for the rows that the DMA kernel leaves over (store and accumulate).
 enum GemmElse { kElseRs, kElseDma, kElseTail };
 
 // The few-row kernel's tile for a product, 0 where the other kernel is faster.
@@ -908,11 +908,11 @@ enum GemmElse { kElseRs, kElseDma, kElseTail };
 //      37.6 / 37.9 / 38.4 / 38.6; gdn_in 200 / 300 / 400 rows 20.8 / 28.0 / 33.3 against 30.2 / 31.0 / 31.6; attn_in
 //      500 / 700 rows 25.6 / 34.1 against 30.5 / 31.4: the lines cross at about 1400 blocks. At K < 512 the waves' sums
 //      weigh more: 3072 x 256 at 640 / 768 rows 11.8 / 14.9 against 13.4 / 13.7, about 1000 blocks.
-//      Against the register-staged kernel, for the rows a wide product leaves over (store / SwiGLU): 5120 x 1024 at 256 /
-//      384 / 512 rows 19.1 / 23.2 / 28.2 against 21.1 / 21.7 / 25.7, gate_up at 256 / 384 rows 23.4 / 31.9 against 23.9 /
-//      27.6, 16,384 x 1024 at 128 rows 25.2 against 22.7, 3072 x 256 at 256 / 384 rows 7.2 / 10.1 against 7.9 / 8.1, 3072 x 512
-//      at 384 / 512 rows 12.5 / 13.5 against 12.5 / 12.9, 4096 x 2048 at 512 / 640 rows 43.8 / 53.5 against 43.3 / 49.7: 900
-//      blocks at K 1024, fewer with shorter rows.
+//      Against the register-staged kernel, for the rows a wide product leaves over: 5120 x 1024 at 256 / 384 / 512 rows
+//      19.1 / 23.2 / 28.2 against 21.1 / 21.7 / 25.7, 16,384 x 1024 at 128 rows 25.2 against 22.7, 3072 x 256 at 256 / 384 rows
+//      7.2 / 10.1 against 7.9 / 8.1, 3072 x 512 at 384 / 512 rows 12.5 / 13.5 against 12.5 / 12.9, 4096 x 2048 at 512 / 640
+//      rows 43.8 / 53.5 against 43.3 / 49.7: 900 blocks at K 1024, fewer with shorter rows. With the SwiGLU epilogue the
+//      first line stays (the register-staged kernel stores single values): an MLP of 6144 rows, 384 left over, 372 against 385.
 //   4  64 x 64, 4 waves: more than one round of tile 2, against the register-staged kernel, while its blocks fit one
 //      round (down 700 / 1000 rows 32.8 / 33.8 against 34.2 / 39.7 for tile 3 and 66.1 / 66.4; not at K < 512, 1024 x 256
 //      at 1024 rows 8.5 against 8.0, bf16 x 7.4 against 6.5).
@@ -1074,7 +1074,8 @@ static int gemm_q8_run(const float* x, int64_t ldx, const int8_t* W, int w_dtype
     if (r != Q35_OK) return r;
     if (Md < M) {
       r = gemm_small_launch<XF>(x + Md * ldx, ldx, W, w_scale, y + Md * ldy, ldy, M - Md, Nd, K, epilogue, gs, pushes,
-                                npush, T, Md, ys, cap, st, gemm_few_tile(M - Md, Nd, K, ldx, xb, kElseTail));
+                                npush, T, Md, ys, cap, st,
+                                gemm_few_tile(M - Md, Nd, K, ldx, xb, epilogue == kGemmSwiglu ? kElseDma : kElseTail));
       if (r != Q35_OK) return r;
     }
     if (Nd < N)

@@ -305,3 +305,5 @@ def test_gemm_q8_left_over_rows(x_form, M, N, K):
     bound = 1.1 * tol[:, 0::2] * (up.abs() + tol[:, 1::2]) + act.abs() * tol[:, 1::2] + 2.0 ** -20 * exp.abs()
     exp[:, 3] += torch.tensor([1.0, -2.0, 0.5]).double()[torch.arange(M) // T]
     assert bool(((a - exp).abs() <= bound + 2.0 ** -23 * exp.abs()).all())
+    b = ops.gemm_q8(xin, q.to(dev), s.to(dev), epilogue="swiglu", pushes=pk, T=T, split_out=True)
+    assert torch.equal(b, ops.split_activations(a.float().to(dev)))  # (the same kernels, whatever the layout of out)
