@@ -1293,7 +1293,7 @@ extern "C" int q35_gated_attn_prefill_cached(const void* q, const void* k_cache,
   __bf16* vt = static_cast<__bf16*>(workspace);
   hipLaunchKernelGGL(attn_vcache_prep_kernel, dim3((unsigned)(max_len / kBN), (unsigned)Hkv, (unsigned)B), dim3(256),
                      0, st, (const __bf16*)v_cache, pos, vt, (int)T, (int)max_len, (int)Hkv);
-  // one item per query block (no key split: the key range depends on the device positions), latest block first
+  // one item per query block (no key runs: this form's workspace has no room for their partials), latest block first
 #define Q35_PFC_LAUNCH(GG)                                                                                        \
   hipLaunchKernelGGL((attn_prefill_kernel<GG, false, false, false>), dim3((unsigned)nblocks), dim3(64 * GG), 0, st,     \
                      (const __bf16*)q, (const __bf16*)k_cache, vt, gate, Hq * kPD, cos, sin, 0, (__bf16*)out,      \

@@ -960,9 +960,10 @@ __global__ __launch_bounds__(kScanThreads, 1) void gdn_pair_scan_kernel(const ch
 //   e^gamma_last,  with T = (I - L)^-1, L[t][s] = -beta_t (k^_t . k^_s) e^(gamma_t - gamma_s) (s < t).
 // Kernel F2, gdn_f32_scan_kernel: 8 blocks per (row, head), one per 16 value columns (4 blocks of 32 columns when 8
 // per (row, head) would exceed the 256 blocks that are resident at once); each carries its 128 x 16 (or 32) fp32
-// state slice in registers (wave w: state rows 32 w .. 32 w + 31) and per chunk computes
+// state slice in the registers of four state waves (wave w: state rows 32 w .. 32 w + 31) and per chunk computes
 //   V = U - W S,   O = Qe S + P V,   S <- e^gamma_last S + Kt V
-// (wave w: positions 16 w .. 16 w + 15 of V and O). The state and V tiles are exchanged through LDS.
+// (state wave w: S, and positions 16 w .. 16 w + 15 of V; four output waves: the same positions of O). The state and V
+// tiles reach the other waves through LDS.
 //
 // Product layout: an operand X[m][k] held row-major feeds the A (or B) side of a 16 x 16 x 4 MFMA group over one
 // 16-wide k chunk as one float4 per lane (X[m][16 c + 4 g .. + 3], m = lane % 16, g = lane / 16), step s using

@@ -31,12 +31,13 @@
 //     the two lanes and turns the activations into whole rows in LDS.
 //   gemm_q8_rs_kernel (the rest: the N = 1024 output and down projections): 2 x 2 waves over BM x 128 tiles, x and W
 //     staged through registers into LDS (split and widened on the way), the next K step's loads issued before the
-//     current step's MFMAs; two blocks per CU.
+//     current step's MFMAs; three blocks per CU with BM 64, two with BM 128.
 // Split input (XS, q35_gemm_q8_split): x arrives already split by its producer, in the same bytes as fp32 x: each
 // group of 8 consecutive inputs of a row is 32 bytes, the 8 bf16 hi parts then the 8 bf16 lo parts (the split above,
-// rounded the same way). Both kernels then skip the split: the DMA kernel copies the 16-byte hi and lo pieces
+// rounded the same way). The kernels then skip the split: the DMA kernel copies the 16-byte hi and lo pieces
 // straight into the planes its A fragments are read from (no fp32 stage, no conversion pass), the register-staged
-// kernel stores the loaded pieces as they are. The products, and so y, are bitwise those of the fp32 input.
+// kernel stores the loaded pieces as they are, the few-row kernel reads them from its stages as fragments. The products,
+// and so y, are bitwise those of the fp32 input.
 // bf16 input (q35_gemm_q8_bf16, the attention output): hi = x exactly and lo = 0, so the few-row and register-staged
 // kernels issue only the hi products (the skipped products are exact zeros): bitwise the product of x.float() wherever the
 // fp32 input runs the same kernel (N < 2048 or K > 2048); for the wide shapes the fp32 input may run the
@@ -647,7 +648,8 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_rs_kernel(const float* __restr
 // touches another row's cache line, about 90 cycles per 1 KB wave load on a CU, 15.9-28 us for the 111-row gate/up.
 // x is re-read by every block of a row panel through L2, which bounds the kernel. The waves' sums meet in LDS, each in
 // its own stage area, and are added in wave order (fixed order, as the tiled kernels).
-// whether the column tiles are dealt to the XCDs (evenly to within an eighth)
+
+// Whether its column tiles are dealt to the XCDs (evenly to within an eighth).
 __host__ __device__ constexpr bool gemm_few_by_xcd(int64_t N, int BN) {
   return (N + BN - 1) / BN % 8 == 0 || (N + BN - 1) / BN >= 64;
 }

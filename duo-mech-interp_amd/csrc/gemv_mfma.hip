@@ -1,8 +1,8 @@
-// The decode GEMV on the matrix core (4 to 8 rows of x, with the tile loop 1 to 8, int8 weights): the products, prologues and epilogues of gemv.hip,
-// whose launcher decides which form runs.
+// The decode GEMV on the matrix core (4 to 8 rows of x, with the tile loop 1 to 8, int8 weights): the products, prologues
+// and epilogues of gemv.hip, whose launcher decides which form runs.
 //
-// The form of gemv.hip spends one FMA per weight and row of x and reads x from LDS for every few rows of W; past three rows of x
-// that sets its time, not the weights' bytes. Here x is split into three bf16 pieces, hi + mid + lo = x exactly (8
+// The form of gemv.hip spends one FMA per weight and row of x and reads x from LDS for every few rows of W; past three
+// rows of x that sets its time, not the weights' bytes. Here x is split into three bf16 pieces, hi + mid + lo = x exactly (8
 // significant bits each, by truncation), int8 weights are exact in bf16, and a v_mfma_f32_16x16x32_bf16 multiplies 16
 // output rows by 16 columns = (piece, row of x): every product is exact and is summed in fp32, where an fp32 FMA chain
 // rounds each partial sum once (error against 64 bits 7e-8 to 1.6e-7 here, 1.1e-7 to 2.2e-7 there). Up to five rows of x
