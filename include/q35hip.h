@@ -142,7 +142,8 @@ int q35_gdn_chunk_prefill(const void* q, const void* k, const void* v, const flo
  *   Needs q35_gated_attn_prefill_workspace_bytes(B, T, Hq, Hkv, D) bytes of workspace (256-byte aligned): the
  *   keys rotated once and the values transposed once ([B, Hkv, T rounded up to 64, D] bf16 each) and, for long
  *   sequences, the fp32 partial results of the query blocks whose keys are split over two work items (combined by
- *   a third kernel). The workspace is overwritten by every call; calls that share one workspace must not overlap.
+ *   a third kernel); where fewer than 256 query blocks run, those of their key runs (at most 512 of up to 133 KB). The
+ *   workspace is overwritten by every call; calls that share one workspace must not overlap.
  */
 size_t q35_gated_attn_prefill_workspace_bytes(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t D);
 int q35_gated_attn_prefill(const void* q, const void* k, const void* v, const void* gate,
@@ -215,8 +216,8 @@ int q35_gated_attn_decode_proj(const float* y, int64_t ldy, const float* q_norm_
  * pos0 + t (pos0 + T <= max_len), bitwise the rows q35_attn_prep writes. out = attention * sigmoid(gate),
  * [B, T, Hq * D] bf16. Limits as q35_gated_attn_prefill (D 256, Hq / Hkv in 1, 2, 4, 8, rot a multiple of 16, at
  * most 64); y, ldy and the norm weights 16-byte aligned; cos, sin [P, rot / 2] fp32 with P >= pos0 + T. Needs
- * q35_gated_attn_prefill_proj_workspace_bytes(B, T, Hq, Hkv, D) bytes of workspace (256-byte aligned); calls that
- * share one workspace must not overlap.
+ * q35_gated_attn_prefill_proj_workspace_bytes(B, T, Hq, Hkv, D) bytes of workspace (256-byte aligned; partials as
+ * for q35_gated_attn_prefill); calls that share one workspace must not overlap.
  */
 size_t q35_gated_attn_prefill_proj_workspace_bytes(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t D);
 int q35_gated_attn_prefill_proj(const float* y, int64_t ldy, const float* q_norm_w, const float* k_norm_w, float eps,
@@ -234,7 +235,8 @@ int q35_gated_attn_prefill_proj(const float* y, int64_t ldy, const float* q_norm
  * pos[b] + T <= max_len), and token t attends to cache keys 0 .. P_b + t. out [B, T, Hq * D] bf16. Limits as
  * q35_gated_attn_prefill_cached (max_len a multiple of 64); y, ldy and the norm weights 16-byte aligned. Needs
  * q35_gated_attn_prefill_cached_proj_workspace_bytes(B, T, Hq, Hkv, D, max_len) bytes of workspace (256-byte
- * aligned); calls that share one workspace must not overlap.
+ * aligned; for caches of at least 12 tiles of 64 keys with room for key runs' partials, at most 256 of 133 KB); calls
+ * that share one workspace must not overlap.
  */
 size_t q35_gated_attn_prefill_cached_proj_workspace_bytes(int64_t B, int64_t T, int64_t Hq, int64_t Hkv, int64_t D,
                                                           int64_t max_len);
